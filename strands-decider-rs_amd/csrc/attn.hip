@@ -2,15 +2,16 @@
 // write (reference: src/kernels.rs:400-448), and causal GQA attention with a sigmoid output gate
 // (reference: src/kernels.rs:453-541).
 //
-// Attention runs on MFMA (k_attn below).  When the query blocks alone cannot fill the GPU (the
-// short question suffix over a long cached prefix), the key range is also split over workgroups
-// and a combine kernel merges the partial (max, sum, acc).  As in the reference, q is pre-scaled
+// Attention runs on MFMA: k_attn for up to 128 rows, k_attn_rows above (attn_plan).  When the query
+// blocks alone cannot fill the GPU (the short question suffix over a long cached prefix), the key range
+// is also split over workgroups and a combine kernel merges the partial (max, sum, acc).  As in the reference, q is pre-scaled
 // by 1/sqrt(hd) and rounded to f16 before the dot products.  The cache is kept in blocks of 32
 // keys, so that the fragment loads of a key block touch whole cache lines: K as [hk][ctx / 32]
 // [hd / 32][32 keys][32 dims] (a load of 16 keys x 8 dims reads pairs of consecutive keys' 64 bytes),
 // V transposed as [hk][ctx / 32][hd][32 keys] (a block's V^T is 16 KB of consecutive bytes).
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 #include "device.h"
@@ -116,6 +117,20 @@ __global__ __launch_bounds__(256) void k_qk_prep(const f16* __restrict__ big, co
 // merges) are in these units.
 constexpr float LOG2E = 1.4426950408889634f;
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Two f32 to packed f16 (round to nearest even), and p minus the low or high half of a packed pair in f32
+// (one v_fma_mix_f32 each, exact: the compiler converts each half on its own otherwise).
+__device__ __forceinline__ uint32_t cvt_pk(float a, float b) { return __builtin_bit_cast(uint32_t, f16x2{(f16)a, (f16)b}); }
+__device__ __forceinline__ float sub_lo(float p, uint32_t h) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(p));
+    return r;
+}
+__device__ __forceinline__ float sub_hi(float p, uint32_t h) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(p));
+    return r;
+}
 
 __device__ __forceinline__ float wave_max16(float v) {  // max over lanes {l, l^16, l^32, l^48}
     v = fmaxf(v, __shfl_xor(v, 16));
@@ -492,6 +507,453 @@ __global__ __launch_bounds__(256) void k_attn(const f16* __restrict__ Q, const f
     }
 }
 
+// The same attention over 32 (query, head) rows per workgroup: NQ = 32 / G queries of all G query
+// heads of one kv head (G = HQ / HK, a power of two), so that a key block feeds 32 rows on
+// v_mfma_f32_32x32x16_f16 where k_attn's feeds 16.  k_attn is bound by the CU's vector memory path (a
+// block is 32 KB per wave, 64 bytes a clock per CU) and by one wave per SIMD waiting in turn for its
+// loads, its softmax and its MFMAs.  This kernel is bound by that path too (2048 clocks for the four
+// waves' blocks, measured 2340 per block beside 1536 of MFMA), for twice the rows, plus about 15 thousand
+// clocks per workgroup of prologue and merge.  On MI355X, 8 query and 2 kv heads: 38.8 us at 2048 rows where
+// k_attn takes 104 us, 18.1 against 39 at 1024, 14.6 against 22.7 at 632; 440 TFLOP/s at 2048.
+//  * Row c of the workgroup is query c % NQ of head kh G + c / NQ; the 4 waves split the keys in blocks
+//    of 32 as in k_attn and merge their states in LDS at the end.
+//  * A wave's block goes straight to LDS (buffer_load_dwordx4 lds, whole cache lines: the 16 KB of K
+//    and of V^T are contiguous in the cache) into a place of the wave's own, so the key loop has no
+//    barrier.  The place holds one block, as 4 + 4 quarters of 4 KB: a quarter is refilled with the next
+//    block's as soon as its fragments have been read.  Rows of 64 bytes (a key's 32 dims of K, a dim's
+//    32 keys of V^T) have their 16-byte pieces at p ^ (row / 4) % 4, so a fragment read (32 rows, two
+//    pieces) meets no bank twice.
+//  * Per block: S^T = K Q^T (keys x rows, 16 MFMAs over the 256 dims in two chains), the softmax per
+//    column, O^T += V^T P^T (8 dim tiles x 2 key slices, P as f16 hi + lo).  The rows of S^T are permuted
+//    so that lane (column, half g) holds keys 16 s + 8 g .. + 7 in registers 8 s ..: P^T's B operand of
+//    slice s as it is.  Block n + 1's S MFMAs run among block n's exponentials.
+//  * The running maximum a row's exponentials are relative to is raised (and O, l rescaled) only when a
+//    block's maximum exceeds it by more than 8: the probabilities then reach at most e^8 = 2981, well inside
+//    f16 (hi + lo keep their relative precision), and the factor cancels in acc / l.  Most blocks skip the rescale.
+//  * Heavy workgroups first: tiles are taken from the last query block down, so the short ones fill the
+//    end; blockIdx.x is the kv head, so with 2 kv heads an XCD's L2 sees one head's keys.
+// Vector-memory accounting (every block issues the same DMAs; past the wave's last block they carry
+// out-of-range offsets, read nothing and write zeros): in the loop the DMAs in flight are block n + 1's
+// K (16), then block n's V (16); reading quarter q leaves the 28 after it, also while the quarters
+// before it are refilled.
+template <int HD, int QRD>
+__global__ __launch_bounds__(256, 1) void k_attn_rows(const f16* __restrict__ Q, const f16* __restrict__ Kc,
+                                                      const f16* __restrict__ Vt, const uint32_t* __restrict__ lu,
+                                                      int L, int HQ, int HK, int stride, int ctx, int ks,
+                                                      const uint32_t* __restrict__ rowt, const f16* __restrict__ big,
+                                                      f16* __restrict__ out, float* __restrict__ pacc,
+                                                      float* __restrict__ pml, const float* __restrict__ qw,
+                                                      const float* __restrict__ rope, int lgq) {
+    static_assert(HD == 256, "attention is written for 256-wide heads");
+    constexpr int NS = HD / 16;   // 16 k steps over the head dimension
+    constexpr int ND = HD / 32;   // 8 output dimension tiles
+    constexpr int KB = 32;        // keys per block
+    constexpr int QB = 4096;      // bytes of a quarter of a wave's K or V^T block
+    constexpr float RAISE = 8.0f;  // the slack of the running maximum
+    // One array per quarter (all 4 waves'), so that the compiler sees that the DMAs into one never alias
+    // the reads of another.  At the end array dt holds the waves' outputs of dim tile dt.
+    __shared__ __align__(1024) uint8_t B0[4 * QB], B1[4 * QB], B2[4 * QB], B3[4 * QB], B4[4 * QB], B5[4 * QB], B6[4 * QB], B7[4 * QB];
+    __shared__ __align__(16) f16 Qs[32][HD + 8];  // the rows' queries, scaled
+    __shared__ float Mm[4][32], Lm[4][32];
+    auto arr = [&](int i) {
+        return i == 0 ? B0 : i == 1 ? B1 : i == 2 ? B2 : i == 3 ? B3 : i == 4 ? B4 : i == 5 ? B5 : i == 6 ? B6 : B7;
+    };
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 31, g = lane >> 5;
+    const int NQ = 1 << lgq;
+    const int kh = blockIdx.x, z = blockIdx.z;
+    const int t0 = (((L + NQ - 1) >> lgq) - 1 - (int)blockIdx.y) * NQ;
+    const int h0 = kh << (5 - lgq);
+    const int nq = min(NQ, L - t0);
+    // The rows' inputs first (they depend on no load): wave w prepares rows 8w .. 8w + 7 in two passes of
+    // 4 (see k_attn), lane (row, part kq) two 8-dim chunks c0, c1; then the epilogue's thread (row ce,
+    // dims 32 dt + 4 ke .. + 3) its output gates.
+    constexpr int RD2 = QRD / 2, NR = RD2 / 8;
+    const int kq = lane & 15;
+    const bool rot = kq < NR;
+    const int c0 = rot ? kq : 2 * kq, c1 = rot ? kq + NR : 2 * kq + 1;
+    int tq[2];
+    f16x8 xv[2][2];
+    float4 wq[2][2], cs4[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int row = 8 * wv + 4 * u + (lane >> 4);
+        tq[u] = t0 + min(row & (NQ - 1), nq - 1);
+        const int hq = h0 + (row >> lgq);
+        const f16* xrow = QRD ? big + (size_t)tq[u] * stride + hq * 2 * HD : Q + ((size_t)hq * L + tq[u]) * HD;
+        xv[u][0] = *reinterpret_cast<const f16x8*>(xrow + 8 * c0);
+        xv[u][1] = *reinterpret_cast<const f16x8*>(xrow + 8 * c1);
+    }
+    if constexpr (QRD != 0) {
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) wq[k][u] = *reinterpret_cast<const float4*>(qw + 8 * (k ? c1 : c0) + 4 * u);
+    }
+    const int ce = tid >> 3, ke = tid & 7;
+    const int te = t0 + min(ce & (NQ - 1), nq - 1), he = h0 + (ce >> lgq);
+    f16x4 gv[ND];
+    {
+        const f16* gp = big + (size_t)te * stride + he * 2 * HD + HD + 4 * ke;
+#pragma unroll
+        for (int u = 0; u < ND; u++) gv[u] = *reinterpret_cast<const f16x4*>(gp + 32 * u);
+    }
+    // row table words, as in k_attn: this lane's query, the tile's first row, and (for the RoPE position)
+    // the queries whose chunks this lane normalizes
+    // (a forward without a table takes a branch of its own: its RoPE rows then wait for no load)
+    const int qi = c & (NQ - 1);
+    uint32_t rwq = 0, rw0 = 0, rpos[2] = {(uint32_t)tq[0], (uint32_t)tq[1]};
+    asm volatile("" ::"s"(big), "s"(qw), "s"(rowt), "s"(Q) : "memory");
+    if (rowt) {
+        const Rsrc rr = make_rsrc(rowt, (uint32_t)L * 4u);
+        rwq = buf_b32(rr, (uint32_t)(t0 + min(qi, nq - 1)) * 4u, 0);
+        rw0 = buf_b32(rr, (uint32_t)t0 * 4u, 0);
+        if constexpr (QRD != 0) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) rpos[u] = buf_b32(rr, (uint32_t)tq[u] * 4u, 0) & 0xFFFFu;
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    const int P = (int)lu[1], Pv = P + (int)lu[6];
+    SGPR_BATCH("s"(P), "s"(Pv), "s"(out), "s"(pacc), "s"(pml));
+    const int nkeys = P + t0 + nq;
+    const int span = ((nkeys + ks - 1) / ks + KB - 1) / KB * KB;
+    const int kbeg = z * span, kend = min(nkeys, kbeg + span);
+    const float scale = 1.0f / sqrtf((float)HD);
+    const int jend = qi < nq ? min(kend, P + t0 + qi + 1) : INT_MIN;
+    if constexpr (QRD != 0) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const float* rp = rope + ((size_t)(P + (int)rpos[u]) * RD2 + 8 * (kq % NR)) * 2;
+#pragma unroll
+            for (int v = 0; v < 4; v++) cs4[u][v] = *reinterpret_cast<const float4*>(rp + 4 * v);
+        }
+        asm volatile("" ::"s"(rope) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int qlo = P + (int)(rwq >> 16), qlo0 = P + (int)(rw0 >> 16);
+
+    const Rsrc rk = make_rsrc(Kc + (size_t)kh * ctx * HD, (uint32_t)ctx * HD * 2u),
+               rv = make_rsrc(Vt + (size_t)kh * HD * ctx, (uint32_t)ctx * HD * 2u);
+    auto next_block = [&](int j) {
+        if (j >= Pv && j + KB <= qlo0) j += ((qlo0 - KB - j) / (4 * KB) + 1) * (4 * KB);
+        return __builtin_amdgcn_readfirstlane(j);
+    };
+    // quarter q of a 16 KB block at byte boff of the cache, 4 KB: lane's 16 bytes of each KB
+    const uint32_t dlane = (uint32_t)((lane >> 2) * 64 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4));
+    auto boff = [&](int j) { return j < kend ? (uint32_t)(j >> 5) * (HD * 64u) : OOB; };
+    auto dma = [&](Rsrc r, int i, uint32_t off) {  // array i: quarter i & 3
+        uint8_t* const dst = arr(i) + wv * QB;
+        buf_lds64(r, dlane, off + (uint32_t)((i & 3) * QB), dst);
+    };
+    // fragment st of K (dims 16 st + 8 g of key kperm of row c), fragment (dt, s) of V^T (keys 16 s + 8 g
+    // of dim 32 dt + c)
+    const int kperm = 16 * (c >> 4) + 8 * ((c >> 2) & 1) + 4 * ((c >> 3) & 1) + (c & 3);
+    const int kfo = kperm * 64 + ((g ^ ((kperm >> 2) & 3)) << 4), vfo = c * 64 + ((g ^ ((c >> 2) & 3)) << 4);
+    auto kfrag = [&](int st) {
+        return *reinterpret_cast<const f16x8*>(arr(st >> 2) + wv * QB + ((st >> 1) & 1) * 2048 + (kfo ^ ((st & 1) << 5)));
+    };
+    auto vfrag = [&](int dt, int k) {
+        return *reinterpret_cast<const f16x8*>(arr(4 + (dt >> 1)) + wv * QB + (dt & 1) * 2048 + (vfo ^ (k << 5)));
+    };
+    f16x8 qf[NS];
+    f32x16 acc[ND];
+#pragma unroll
+    for (int dt = 0; dt < ND; dt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[dt][i] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    int j = next_block(kbeg + wv * KB);
+    {
+        const uint32_t b = boff(j);
+#pragma unroll
+        for (int q = 0; q < 4; q++) dma(rk, q, b);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        f16x8 q8[2];
+        if constexpr (QRD == 0) {
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) q8[k][e] = (f16)((float)xv[u][k][e] * scale);
+        } else {
+            float x[2][8], sp[2] = {0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    x[k][e] = (float)xv[u][k][e];
+                    sp[k] += x[k][e] * x[k][e];
+                }
+            float ss = sp[0] + sp[1];
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o);
+            const float inv = 1.0f / sqrtf(ss / (float)HD + 1e-6f);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float w8[8] = {wq[k][0].x, wq[k][0].y, wq[k][0].z, wq[k][0].w,
+                                     wq[k][1].x, wq[k][1].y, wq[k][1].z, wq[k][1].w};
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[k][e] = x[k][e] * inv * w8[e];
+            }
+            const float cs[16] = {cs4[u][0].x, cs4[u][0].y, cs4[u][0].z, cs4[u][0].w, cs4[u][1].x, cs4[u][1].y,
+                                  cs4[u][1].z, cs4[u][1].w, cs4[u][2].x, cs4[u][2].y, cs4[u][2].z, cs4[u][2].w,
+                                  cs4[u][3].x, cs4[u][3].y, cs4[u][3].z, cs4[u][3].w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float cc = cs[2 * e], sn = cs[2 * e + 1], a = x[0][e], bb = x[1][e];
+                const float lo = rot ? a * cc - bb * sn : a, hi = rot ? bb * cc + a * sn : bb;
+                q8[0][e] = (f16)((float)(f16)lo * scale);
+                q8[1][e] = (f16)((float)(f16)hi * scale);
+            }
+        }
+        const int row = 8 * wv + 4 * u + (lane >> 4);
+        *reinterpret_cast<f16x8*>(&Qs[row][8 * c0]) = q8[0];
+        *reinterpret_cast<f16x8*>(&Qs[row][8 * c1]) = q8[1];
+    }
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        qf[s] = *reinterpret_cast<const f16x8*>(&Qs[c][s * 16 + g * 8]);
+        asm("" : "+a"(qf[s]));  // kept in AGPRs, which an MFMA reads as it reads VGPRs
+    }
+
+    // masked scores (unscaled, natural units) and their column maximum over both lane halves
+    auto mask_max = [&](f32x16& s, int j0) {
+        const bool open = j0 + KB <= kend && j0 + KB <= P + t0 + 1 && (!rowt || j0 + KB <= Pv);
+        if (!open) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int key = j0 + 16 * (i >> 3) + 8 * g + (i & 7);
+                const bool keep = (key < jend) & ((key < Pv) | (key >= qlo));
+                s[i] = keep ? s[i] : -INFINITY;
+            }
+        }
+        float t = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) t = fmaxf(t, s[i]);
+        // (the swap's halves through scalars: a bit cast of a vector's element reads element 0)
+        const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, t), __builtin_bit_cast(uint32_t, t), false, false);
+        const uint32_t lo = sw[0], hi = sw[1];
+        return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+    };
+    // The block's probabilities 2^(s log2 e + nm) and their split into f16 hi + lo, pair by pair: pexp
+    // exponentiates elements 2u, 2u + 1, psplit adds them to the row sum and packs them.
+    f16x8 ph[2], pl[2];
+    float pe[16];
+    auto pexp = [&](const f32x16& s, int u, float nm) {
+        pe[2 * u] = exp2_fast(__builtin_fmaf(s[2 * u], LOG2E, nm));
+        pe[2 * u + 1] = exp2_fast(__builtin_fmaf(s[2 * u + 1], LOG2E, nm));
+    };
+    auto psplit = [&](int u) {
+        const float p0 = pe[2 * u], p1 = pe[2 * u + 1];
+        const uint32_t h2 = cvt_pk(p0, p1);
+        const f16x2 hi = __builtin_bit_cast(f16x2, h2), lo = __builtin_bit_cast(f16x2, cvt_pk(sub_lo(p0, h2), sub_hi(p1, h2)));
+        l_run += p0;
+        l_run += p1;
+        ph[u >> 2][(2 * u) & 7] = hi[0];
+        ph[u >> 2][(2 * u + 1) & 7] = hi[1];
+        pl[u >> 2][(2 * u) & 7] = lo[0];
+        pl[u >> 2][(2 * u + 1) & 7] = lo[1];
+    };
+    auto raise = [&](float tmax) {
+        if (!__any(tmax > m_run + RAISE)) return;
+        const float m_new = fmaxf(m_run, tmax);
+        const float alpha = m_run == -INFINITY ? 0.f : exp2_fast((m_run - m_new) * LOG2E);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[dt][i] *= alpha;
+    };
+    // The loop's unit is a quarter: its fragments were read during the quarter before, and while its MFMAs
+    // run the next quarter's are (once its DMAs have landed: WAIT leaves the DMAs after it in flight); then
+    // the quarter itself is refilled.  `mid(e)` is VALU work beside MFMA e.
+    f16x8 fr[2][4];
+    auto read_k = [&](int q) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) fr[q & 1][e] = kfrag(4 * q + e);
+    };
+    auto read_v = [&](int q) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) fr[q & 1][e] = vfrag(2 * q + (e & 1), e >> 1);
+    };
+    auto k_quarter = [&](f32x16& s, int q, auto mid) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[q & 1][e], qf[4 * q + e], s, 0, 0, 0);
+            mid(4 * q + e);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto v_quarter = [&](int q) {
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+                acc[2 * q + d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[q & 1][e + d], ph[e >> 1], acc[2 * q + d], 0, 0, 0);
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+                acc[2 * q + d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[q & 1][e + d], pl[e >> 1], acc[2 * q + d], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr int W24 = vmcnt_imm(24), W12 = vmcnt_imm(12), W8 = vmcnt_imm(8), W4 = vmcnt_imm(4), W0 = vmcnt_imm(0);
+    if (j < kend) {
+        int jn = next_block(j + 4 * KB);
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
+        {
+            // the first block: its K alone is in flight, then block jn's behind it, then its own V
+            const uint32_t kn = boff(jn), b = boff(j);
+            wait_loads<W12>();
+            read_k(0);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (q < 3) {
+                    wait_loads<W8>();
+                    read_k(q + 1);
+                }
+                k_quarter(s, q, [](int) {});
+                dma(rk, q, kn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) dma(rv, 4 + q, b);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (jn < kend) {
+            wait_loads<vmcnt_imm(28)>();
+            read_k(0);
+        }
+        float tmax = mask_max(s, j);
+        while (jn < kend) {
+            raise(tmax);
+            const int j2 = next_block(jn + 4 * KB);
+            const uint32_t kn = boff(j2), vn = boff(jn);
+            const float nm = m_run == -INFINITY ? 0.f : m_run * -LOG2E;
+            f32x16 s2;
+#pragma unroll
+            for (int i = 0; i < 16; i++) s2[i] = 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                wait_loads<W24>();
+                if (q < 3) read_k(q + 1);
+                else read_v(0);
+                k_quarter(s2, q, [&](int st) {
+                    if (st % 2 == 0) pexp(s, st >> 1, nm);
+                    else psplit(st >> 1);
+                });
+                dma(rk, q, kn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                wait_loads<W24>();
+                if (q < 3) read_v(q + 1);
+                else read_k(0);  // block j2's; past the wave's last block it reads zeros, for nothing
+                v_quarter(q);
+                dma(rv, 4 + q, vn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            s = s2;
+            tmax = mask_max(s, jn);
+            j = jn;
+            jn = j2;
+        }
+        // the last block: its V alone is to be waited for
+        wait_loads<W12>();
+        read_v(0);
+        raise(tmax);
+        const float nm = m_run == -INFINITY ? 0.f : m_run * -LOG2E;
+#pragma unroll
+        for (int u = 0; u < 8; u++) pexp(s, u, nm);
+#pragma unroll
+        for (int u = 0; u < 8; u++) psplit(u);
+        wait_loads<W8>();
+        read_v(1);
+        v_quarter(0);
+        wait_loads<W4>();
+        read_v(2);
+        v_quarter(1);
+        wait_loads<W0>();
+        read_v(3);
+        v_quarter(2);
+        v_quarter(3);
+    }
+    wait_loads<vmcnt_imm(0)>();  // every DMA has landed before the arrays take the outputs
+    l_run += __shfl_xor(l_run, 32);
+    // merge the 4 waves: acc[dt][i] is O[row c][dim 32 dt + 8 (i / 4) + 4 g + i % 4]; array dt, wave w's
+    // part: rows of 128 bytes, 16-byte chunk k (dims 4k .. 4k + 3 of the tile) at k ^ row % 8
+#pragma unroll
+    for (int dt = 0; dt < ND; dt++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            *reinterpret_cast<f32x4*>(arr(dt) + wv * QB + c * 128 + (((2 * q + g) ^ (c & 7)) << 4)) =
+                f32x4{acc[dt][4 * q], acc[dt][4 * q + 1], acc[dt][4 * q + 2], acc[dt][4 * q + 3]};
+    if (g == 0) {
+        Mm[wv][c] = m_run * LOG2E;
+        Lm[wv][c] = l_run;
+    }
+    lds_barrier();
+    // every thread merges its row's states itself (8 LDS words, no second barrier)
+    float mq = -INFINITY, lq = 0.f, fw[4];
+    {
+        float mw[4], lw[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) mw[w] = Mm[w][ce], lw[w] = Lm[w][ce];
+#pragma unroll
+        for (int w = 0; w < 4; w++) mq = lw[w] > 0.f ? fmaxf(mq, mw[w]) : mq;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            fw[w] = lw[w] > 0.f ? exp2_fast(mw[w] - mq) : 0.f;
+            lq += lw[w] * fw[w];
+        }
+    }
+    // thread (ce, ke): the 4 waves' outputs summed in wave order
+    f32x4 av[ND];
+#pragma unroll
+    for (int dt = 0; dt < ND; dt++) av[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const float f = fw[w];
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(arr(dt) + w * QB + ce * 128 + ((ke ^ (ce & 7)) << 4));
+#pragma unroll
+            for (int e = 0; e < 4; e++) av[dt][e] += v[e] * f;
+        }
+    }
+    if ((ce & (NQ - 1)) >= nq) return;
+    if (ks == 1) {
+        const float inv_l = 1.0f / lq;
+        f16* op = out + (size_t)te * HQ * HD + he * HD + 4 * ke;
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++) {
+            f16x4 o4;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((float)gv[dt][e] * -LOG2E));
+                o4[e] = (f16)(av[dt][e] * inv_l * sg);
+            }
+            *reinterpret_cast<f16x4*>(op + 32 * dt) = o4;
+        }
+    } else {
+        const size_t r = ((size_t)z * L + te) * HQ + he;
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++) *reinterpret_cast<f32x4*>(pacc + r * HD + 32 * dt + 4 * ke) = av[dt];
+        if (ke == 0) {
+            pml[r * 2] = mq;
+            pml[r * 2 + 1] = lq;
+        }
+    }
+}
+
 template <int HD>
 __global__ __launch_bounds__(HD) void k_attn_combine(const float* __restrict__ pacc, const float* __restrict__ pml,
                                                      const f16* __restrict__ big, f16* __restrict__ out, int L, int ks,
@@ -542,24 +1004,56 @@ void qk_prep(const f16* big, const AttnShape& s, const float* qw, const float* k
 // Workspace (floats) the key-split path needs for up to `rows` query rows.
 size_t attn_ws_floats(int rows, const AttnShape& s) { return (size_t)ATTN_KS_MAX * rows * s.HQ * (s.HD + 2); }
 
+// Which kernel, and how many key splits, for L rows (prefix: the keys include a cached prefix; without one
+// they are the rows themselves).  The splits are fixed when a plan is captured, whatever the prefix's length.
+// qk_prep + attention + combine on MI355X at 8 query and 2 kv heads, us, k_attn against k_attn_rows:
+//   rows + prefix   64 + 512   120 + 512   200 + 512   250 + 2048   256 + 0   512 + 0   1024 + 0   2048 + 0
+//   k_attn          17.0       18.7        27.8        32.3         19.1      20.2      47.9       119
+//   k_attn_rows     18.4       19.3-20.6   22.3        29.4         16.1      19.0      26.7       51.1
+// A tile of 32 (query, head) rows has half as many workgroups as k_attn's 16 queries of a head, so up to 128
+// rows (64 of k_attn's tiles) the latter's shorter chains win.
+//  * k_attn splits the keys while its grid stays within one workgroup per CU (70 rows: 18.2 us in 4 splits,
+//    21.0 in 8).
+//  * k_attn_rows up to 256 rows splits them only over a prefix, in 4 up to 48 tiles (200 + 2048: 25.2 us in 4
+//    splits, 28.3 in 2, 33.0 in 1; 128 + 512: 19.3 / 19.5 / 18.3) and in 2 up to 64 (250 + 512: 24.1 / 23.2 /
+//    20.5, + 2048: 26.7 / 29.4 / 33.4).
+AttnPlan attn_plan(int L, const AttnShape& s, bool prefix) {
+    const int G = s.HQ / s.HK;
+    AttnPlan p;
+    p.rows = L > 128 && G <= 32 && (G & (G - 1)) == 0;
+    if (L > ATTN_SPLIT_ROWS) return p;
+    if (p.rows) {
+        const int tiles = (L * G + 31) / 32 * s.HK;
+        p.ks = !prefix || tiles > 64 ? 1 : tiles > 48 ? 2 : 4;
+    } else {
+        const int tiles = (L + BQ - 1) / BQ * s.HQ;
+        while (p.ks < ATTN_KS_MAX && tiles * p.ks * 2 <= 256) p.ks *= 2;
+    }
+    return p;
+}
+
 void attention_split(const f16* Q, const f16* Kc, const f16* Vc, const f16* big, const AttnShape& s, int L,
-                     const uint32_t* lu, const Segs& sg, int ks, float* ws, f16* out, hipStream_t st, const float* qw,
-                     const float* rope) {
+                     const uint32_t* lu, const Segs& sg, const AttnPlan& p, float* ws, f16* out, hipStream_t st,
+                     const float* qw, const float* rope) {
     SD_CHECK(s.HD == 256 && s.HQ % s.HK == 0, "attention: unsupported head shape");
     SD_CHECK(Q || (qw && rope && s.RD == 64), "attention: the fused query norm and RoPE take rotary_dim 64");
-    SD_CHECK(ks >= 1 && ks <= ATTN_KS_MAX, "attention: 1 to 8 key splits");
-    const int nb = (L + BQ - 1) / BQ;
+    SD_CHECK(p.ks >= 1 && p.ks <= ATTN_KS_MAX, "attention: 1 to 8 key splits");
     float* pacc = ws;
-    float* pml = ws + (size_t)ks * L * s.HQ * s.HD;
-    if (Q)
-        hipLaunchKernelGGL((k_attn<256, 0>), dim3(nb, s.HQ, ks), dim3(256), 0, st, Q, Kc, Vc, lu, L, s.HQ, s.HK, s.stride,
-                           s.ctx, ks, sg.row, big, out, pacc, pml, qw, rope, s.RD);
-    else
-        hipLaunchKernelGGL((k_attn<256, 64>), dim3(nb, s.HQ, ks), dim3(256), 0, st, Q, Kc, Vc, lu, L, s.HQ, s.HK, s.stride,
-                           s.ctx, ks, sg.row, big, out, pacc, pml, qw, rope, s.RD);
+    float* pml = ws + (size_t)p.ks * L * s.HQ * s.HD;
+    const int G = s.HQ / s.HK;
+    if (p.rows) {
+        SD_CHECK(G <= 32 && (G & (G - 1)) == 0, "attention: a tile of 32 rows takes a power of two of query heads");
+        const auto f = Q ? k_attn_rows<256, 0> : k_attn_rows<256, 64>;
+        hipLaunchKernelGGL(f, dim3(s.HK, (L * G + 31) / 32, p.ks), dim3(256), 0, st, Q, Kc, Vc, lu, L, s.HQ, s.HK, s.stride,
+                           s.ctx, p.ks, sg.row, big, out, pacc, pml, qw, rope, 5 - __builtin_ctz((unsigned)G));
+    } else {
+        const auto f = Q ? k_attn<256, 0> : k_attn<256, 64>;
+        hipLaunchKernelGGL(f, dim3((L + BQ - 1) / BQ, s.HQ, p.ks), dim3(256), 0, st, Q, Kc, Vc, lu, L, s.HQ, s.HK, s.stride,
+                           s.ctx, p.ks, sg.row, big, out, pacc, pml, qw, rope, s.RD);
+    }
     launched("attn");
-    if (ks > 1) {
-        hipLaunchKernelGGL(k_attn_combine<256>, dim3(L, s.HQ), dim3(256), 0, st, pacc, pml, big, out, L, ks, s.HQ,
+    if (p.ks > 1) {
+        hipLaunchKernelGGL(k_attn_combine<256>, dim3(L, s.HQ), dim3(256), 0, st, pacc, pml, big, out, L, p.ks, s.HQ,
                            s.stride);
         launched("attn_combine");
     }

@@ -560,11 +560,7 @@ int sd_op_attention(const void* big, int stride, const void* qw, const void* kw,
         if (ctx % 32) throw sd::Error("sd_op_attention: ctx must be a multiple of 32");
         if (HK < 1 || HQ % HK) throw sd::Error("sd_op_attention: q heads must be a multiple of kv heads");
         const sd::AttnShape as{HQ, HK, HD, RD, stride, ctx};
-        // the engine's key split: query blocks of 16 that cannot fill the chip split the keys too
-        const int nb = (L + 15) / 16;
-        int ks = 1;
-        if (L <= 256)
-            while (ks < 8 && nb * HQ * ks < 256) ks *= 2;
+        const sd::AttnPlan ap = sd::attn_plan(L, as, P > 0);  // the engine's
         OpWs& w = op_ws();
         std::lock_guard<std::mutex> lock(w.mu);
         const hipStream_t st = static_cast<hipStream_t>(stream);
@@ -578,7 +574,7 @@ int sd_op_attention(const void* big, int stride, const void* qw, const void* kw,
         // rotary_dim 64: the attention normalizes and rotates the queries itself, as in the engine (Q
         // is still written above for the caller)
         sd::attention_split(RD == 64 ? nullptr : static_cast<const sd::f16*>(Q), static_cast<const sd::f16*>(Kc),
-                            static_cast<const sd::f16*>(Vt), static_cast<const sd::f16*>(big), as, L, lu, sd::Segs{}, ks,
+                            static_cast<const sd::f16*>(Vt), static_cast<const sd::f16*>(big), as, L, lu, sd::Segs{}, ap,
                             reinterpret_cast<float*>(static_cast<uint8_t*>(w.attn) + 256), static_cast<sd::f16*>(out), st,
                             static_cast<const float*>(qw), static_cast<const float*>(rope));
     });

@@ -240,12 +240,20 @@ struct AttnShape {
 void qk_prep(const f16* big, const AttnShape& s, const float* qw, const float* kw, const float* rope, int L,
              const uint32_t* lu, const Segs& sg, f16* Q, f16* Kc, f16* Vc, hipStream_t st);
 // Workspace (floats) of the key-split path for up to `rows` query rows and 8 splits.
+// How the attention of L query rows runs: the kernel (32 rows of all heads of a kv head per workgroup, or 16
+// queries of one head) and its key splits.  Only up to ATTN_SPLIT_ROWS rows split their keys.
+constexpr int ATTN_SPLIT_ROWS = 256;
+struct AttnPlan {
+    bool rows = false;
+    int ks = 1;
+};
+AttnPlan attn_plan(int L, const AttnShape& s, bool prefix);
 size_t attn_ws_floats(int rows, const AttnShape& s);
-// ks = number of key splits (1: no workspace needed; ks > 1 needs rows = L in the workspace).
+// p.ks = number of key splits (1: no workspace needed; ks > 1 needs rows = L in the workspace).
 // Row r attends the prefix (cache rows < P) and its own sequence up to itself.
 // Q null: each workgroup computes its queries' RMSNorm (qw) and RoPE (rope, rotary_dim 64) from big.
 void attention_split(const f16* Q, const f16* Kc, const f16* Vc, const f16* big, const AttnShape& s, int L,
-                     const uint32_t* lu, const Segs& sg, int ks, float* ws, f16* out, hipStream_t st,
+                     const uint32_t* lu, const Segs& sg, const AttnPlan& p, float* ws, f16* out, hipStream_t st,
                      const float* qw = nullptr, const float* rope = nullptr);
 
 }  // namespace sd

@@ -44,6 +44,14 @@ __device__ __forceinline__ Rsrc make_rsrc(const void* base, uint32_t bytes) {
 __device__ __forceinline__ void buf_lds16(Rsrc r, uint32_t voff, uint32_t soff, void* lds) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 0, 0);
 }
+// Four of them, 1 KB apart on both sides (the instruction's immediate offset moves the buffer and the LDS
+// address alike, so they share one scalar offset and one LDS base).
+__device__ __forceinline__ void buf_lds64(Rsrc r, uint32_t voff, uint32_t soff, void* lds) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 1024, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 2048, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 3072, 0);
+}
 __device__ __forceinline__ u32x4 buf_b128(Rsrc r, uint32_t voff, uint32_t soff) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
@@ -67,6 +75,7 @@ __device__ __forceinline__ void buf_st32(Rsrc r, uint32_t voff, uint32_t soff, u
 struct Rsrc {};
 __device__ inline Rsrc make_rsrc(const void*, uint32_t) { return {}; }
 __device__ inline void buf_lds16(Rsrc, uint32_t, uint32_t, void*) {}
+__device__ inline void buf_lds64(Rsrc, uint32_t, uint32_t, void*) {}
 __device__ inline u32x4 buf_b128(Rsrc, uint32_t, uint32_t) { return u32x4{}; }
 __device__ inline uint32_t buf_b16(Rsrc, uint32_t, uint32_t) { return 0; }
 __device__ inline u32x3 buf_b96(Rsrc, uint32_t, uint32_t) { return u32x3{}; }

@@ -523,7 +523,7 @@ void Engine::ensure_pool(int l) {
         (size_t)cfg.hq * cap * cfg.hd * 2,             // q
         (size_t)cap * cfg.d * 4,                       // out
         gdn_ws_bytes(cap, gs),                         // GDN chunk workspace
-        attn_ws_floats(std::min(cap, 256), as) * 4,    // attention key-split workspace
+        attn_ws_floats(std::min(cap, ATTN_SPLIT_ROWS), as) * 4,    // attention key-split workspace
         ypart * 4,                                     // split-K partials of y
         gpart * 4,                                     // split-K partials of gate_up
         (size_t)cap * cfg.d * 4,                       // xc: a compact last layer's residual rows
@@ -567,7 +567,7 @@ void Engine::ensure_pool(int l) {
     pool.out = (float*)ptrs[10];
     gdn_ws_carve(ptrs[11], cap, gs, pool.gdn);
     pool.attn_ws = (float*)ptrs[12];
-    pool.attn_rows = std::min(cap, 256);
+    pool.attn_rows = std::min(cap, ATTN_SPLIT_ROWS);
     pool.ypart = (float*)ptrs[13];
     pool.ypart_elems = ypart;
     pool.gpart = (float*)ptrs[14];
@@ -629,7 +629,7 @@ YIn Engine::mm_y(std::vector<Step>& steps, const char* label, const f16* A, cons
     return y;
 }
 
-Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, int rows_read) {
+Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, int rows_read, bool prefix) {
     // A forward that reads at most half its rows runs its last layer's tail (after the token mixer:
     // o_proj or out_proj, the residual add + norm, the MLP) on the read rows only, gathered into a
     // compact block; the final norm then reads them there.  The mixer itself runs on every row (its
@@ -638,7 +638,10 @@ Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, 
                                 layers.back().kind != SD_ADAPTER
                             ? rows_read
                             : 0;
-    const uint64_t key = (uint64_t)(cache_only ? 1u : 0u) << 63 | (uint64_t)compact << 46 | (uint64_t)tree << 32 |
+    // the attention's plan: the prefix bit is part of the key only where it changes it
+    const AttnShape head{cfg.hq, cfg.hk, cfg.hd, cfg.rd, 0, SD_CONTEXT};
+    const bool split_bit = !attn_layers.empty() && prefix && attn_plan(L, head, true).ks != attn_plan(L, head, false).ks;
+    const uint64_t key = (uint64_t)(cache_only ? 1u : 0u) << 63 | (uint64_t)(split_bit ? 1u : 0u) << 62 | (uint64_t)compact << 46 | (uint64_t)tree << 32 |
                          (uint64_t)L << 8 | (uint64_t)nseq << 1 | (short_seqs ? 1u : 0u);
     auto it = plans.find(key);
     if (it != plans.end()) {
@@ -784,12 +787,10 @@ Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, 
                 qk_prep(P.big, as, W.q_norm, W.k_norm, rp, L, luv, sg, qbuf, W.kc, W.vc, s);
             }});
             if (cache_end) break;
-            const int nb = (L + 15) / 16;
-            int ks = 1;
-            if (L <= P.attn_rows)
-                while (ks < 8 && nb * cfg.hq * ks < 256) ks *= 2;
+            const AttnPlan ap = attn_plan(L, as, split_bit);
+            SD_CHECK(ap.ks == 1 || L <= P.attn_rows, "attention: the key-split workspace is too small");
             steps.push_back({"attn", [=](hipStream_t s) {
-                attention_split(qbuf, W.kc, W.vc, P.big, as, L, luv, sg, ks, P.attn_ws, P.o, s, W.q_norm, rp);
+                attention_split(qbuf, W.kc, W.vc, P.big, as, L, luv, sg, ap, P.attn_ws, P.o, s, W.q_norm, rp);
             }});
             if (tail_c) {
                 const size_t ob = (size_t)W.o_proj.K * 2, xb = (size_t)d * 4;
@@ -976,7 +977,7 @@ void Engine::forward(const uint32_t* ids, size_t n, const size_t* rows, size_t n
     const int L = (int)n;
     SD_CHECK(n_rows <= SD_CONTEXT, "at most 4096 hidden rows per forward");
     ensure_pool(std::max(L, (int)n_rows));  // the row tables and outputs hold n_rows entries
-    Plan& pl = plan(L, 0, false, 0, n_rows == 0, (int)n_rows);
+    Plan& pl = plan(L, 0, false, 0, n_rows == 0, (int)n_rows, cache != nullptr);
     upload(ids, n, rows, n_rows, P, cache != nullptr, 0, 0, cache);
     restore(cache, P);
     launch_and_read(pl, n_rows, timed);
@@ -1047,7 +1048,7 @@ Plan& Engine::prepare_batch(const uint32_t* ids, const size_t* lens, size_t nseq
     const int L = (int)n;
     SD_CHECK(n_rows <= SD_CONTEXT, "at most 4096 hidden rows per forward");
     ensure_pool(std::max(L, (int)n_rows));  // the row tables and outputs hold n_rows entries
-    Plan& pl = plan(L, (int)nseq, any_short, 0, false, (int)n_rows);
+    Plan& pl = plan(L, (int)nseq, any_short, 0, false, (int)n_rows, cache != nullptr);
     // sequence tables (see Segs): rows, chunks of <= 64 rows inside each sequence, sequences
     uint32_t* rowt = reinterpret_cast<uint32_t*>(up_h + pool.off_seg_row);
     uint32_t* chunkt = reinterpret_cast<uint32_t*>(up_h + pool.off_seg_chunk);
@@ -1305,7 +1306,7 @@ size_t Engine::trace(const uint32_t* ids, size_t n, const Snapshot* cache, const
         if (rows[r] >= n) throw Error("row " + std::to_string(rows[r]) + " out of range for " + std::to_string(n) + " tokens");
     const int L = (int)n;
     ensure_pool(L);
-    Plan& pl = plan(L);
+    Plan& pl = plan(L, 0, false, 0, false, 0, cache != nullptr);
     upload(ids, n, nullptr, 0, P, cache != nullptr, 0, 0, cache);
     restore(cache, P);
     const size_t d = (size_t)cfg.d;

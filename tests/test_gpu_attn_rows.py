@@ -1,0 +1,78 @@
+"""The attention kernel that takes 32 (query, head) rows per workgroup (more than 128 rows, a power of two
+of query heads per kv head), against the CPU oracle: edges of its tiles and key blocks, every group size
+it takes, both query paths, scores that raise the running maximum block after block, and the group sizes
+it leaves to the other kernel."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+I = ctypes.c_int
+HD, CTX = 256, 4096
+
+
+def dev(a):
+    a = np.ascontiguousarray(a)
+    return torch.from_numpy(a.view(np.uint8).reshape(-1).copy()).cuda()
+
+
+def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0):
+    """P prefix rows straight in the cache, then L rows; out within 2 f16 ulp + 1e-3 of the oracle (scores,
+    softmax and P V in f32 against the oracle's f64 softmax: the bound of the other attention tests)."""
+    from conftest import f16_ulp
+    rng = np.random.default_rng(seed)
+    qw = (gain * (1 + 0.1 * rng.standard_normal(HD))).astype(np.float32)
+    kw = (1 + 0.1 * rng.standard_normal(HD)).astype(np.float32)
+    rope = o.rope_table(rd, 1e7)
+    stride = 2 * hq * HD + 2 * hk * HD
+    big = rng.standard_normal((L, stride)).astype(np.float16)
+    oK, oV = np.zeros((hk, CTX, HD), np.uint16), np.zeros((hk, CTX, HD), np.uint16)
+    oK[:, :P] = rng.standard_normal((hk, P, HD)).astype(np.float16).view(np.uint16)
+    oV[:, :P] = rng.standard_normal((hk, P, HD)).astype(np.float16).view(np.uint16)
+    dK = dev(oK.reshape(hk, CTX // 32, 32, HD // 32, 32).transpose(0, 1, 3, 2, 4))
+    dV = dev(oV.reshape(hk, CTX // 32, 32, HD).transpose(0, 1, 3, 2))
+    dbig, dqw, dkw, drope = dev(big), dev(qw), dev(kw), dev(rope)
+    dQ = torch.zeros(hq * L * HD * 2, dtype=torch.uint8, device="cuda")
+    dout = torch.zeros(L * hq * HD * 2, dtype=torch.uint8, device="cuda")
+    sdamd.op_attention(dbig.data_ptr(), stride, dqw.data_ptr(), dkw.data_ptr(), drope.data_ptr(), L, P, hq, hk, HD, rd,
+                       dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), CTX, dout.data_ptr())
+    torch.cuda.synchronize()
+    Q = np.empty((hq, L, HD), np.uint16)
+    o.lib().or_qk_prep(o.P(big.view(np.uint16)), I(stride), o.P(qw), o.P(kw), o.P(rope), I(L), I(P), I(CTX), I(hq),
+                       I(hk), I(HD), I(rd), o.P(Q), o.P(oK), o.P(oV))
+    out = np.empty((L, hq * HD), np.uint16)
+    o.lib().or_attn(o.P(Q), o.P(oK), o.P(oV), o.P(big.view(np.uint16)), I(stride), I(L), I(P), I(CTX), I(hq), I(hk),
+                    I(HD), o.P(out))
+    got = dout.cpu().numpy().view(np.float16).reshape(L, hq * HD).astype(np.float32)
+    want = o.h2f(out)
+    # a large gain on q: the 1-ulp f16 difference of a query (2^-11) moves its scores (up to ~100) by ~0.05,
+    # which is a factor e^0.05 between two keys' weights
+    extra = 1e-3 if gain == 1.0 else 5e-2
+    bad = np.abs(got - want) > 2.0 * f16_ulp(want) + extra
+    assert not bad.any(), (f"L={L} P={P} heads {hq}/{hk}: {int(bad.sum())} outputs off, "
+                           f"max {np.abs(got - want).max():.3g}")
+
+
+@pytest.mark.parametrize("L,P", [(129, 0), (136, 31), (150, 0), (159, 64), (193, 33), (257, 95), (300, 0), (513, 700)])
+def test_rows_kernel_edges(sdamd, oracle, L, P):
+    """Ragged last tiles (8 queries each), prefixes that end inside a 32-key block, splits of 1, 2 and 4."""
+    check(sdamd, oracle, L + P, 8, 2, L, P)
+
+
+@pytest.mark.parametrize("hq,hk", [(2, 2), (4, 2), (8, 1), (16, 1), (6, 2)])
+def test_rows_kernel_groups(sdamd, oracle, hq, hk):
+    """1, 2, 8 and 16 query heads per kv head (32, 16, 4 and 2 queries per tile); 3 take the other kernel."""
+    check(sdamd, oracle, 7 * hq + hk, hq, hk, 141, 50)
+
+
+def test_rows_kernel_reads_prepared_queries(sdamd, oracle):
+    """rotary_dim 32: the queries come from qk_prep's buffer."""
+    check(sdamd, oracle, 5, 8, 2, 170, 40, rd=32)
+
+
+def test_rows_kernel_raises_its_maximum(sdamd, oracle):
+    """Queries scaled by 12: scores of a standard deviation of 12 in the exponent, so the running maximum
+    rises by more than the kernel's slack again and again."""
+    check(sdamd, oracle, 9, 8, 2, 400, 100, gain=12.0)
