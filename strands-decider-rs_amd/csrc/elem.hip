@@ -76,6 +76,10 @@ __global__ __launch_bounds__(256) void k_add_norm(float* __restrict__ x, const f
                     const float4 p4 = *reinterpret_cast<const float4*>(yp + z * slot + row * d + c);
                     part[i][z] = p4.x, part[i + 1][z] = p4.y, part[i + 2][z] = p4.z, part[i + 3][z] = p4.w;
                 }
+            } else if (y && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
+                const f16x4 y4 = *reinterpret_cast<const f16x4*>(y + row * d + c);
+#pragma unroll
+                for (int u = 0; u < 4; u++) part[i + u][0] = (float)y4[u];
             } else {
 #pragma unroll
                 for (int u = 0; u < 4; u++) part[i + u][0] = y ? (float)y[row * d + c + u] : 0.f;

@@ -619,10 +619,19 @@ YIn Engine::mm_y(std::vector<Step>& steps, const char* label, const f16* A, cons
     const GemmPlan gp = gemm_w4_plan(L, m.N, m.K, exact, true, pool.ypart_elems);
     const int cfg_ = gp.cfg, ks = gp.ks;
     float* part = pool.ypart;
+    YIn y;
+    if (ks == 1) {
+        // unsplit: the f16 the add + norm would round its only slot to, at half the bytes of the slot
+        f16* const out = pool.y;
+        steps.push_back({label, [=](hipStream_t s) {
+            gemm_w4(A, m.q, m.s, out, nullptr, L, m.N, m.K, exact, 1, s, cfg_, m.tiled);
+        }});
+        y.y16 = out;
+        return y;
+    }
     steps.push_back({label, [=](hipStream_t s) {
         gemm_w4(A, m.q, m.s, nullptr, part, L, m.N, m.K, exact, ks, s, cfg_, m.tiled);
     }});
-    YIn y;
     y.yp = part;
     y.ks = ks;
     y.slot = (size_t)L * m.N;
@@ -803,15 +812,15 @@ Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, 
             steps.push_back({"norm", [=](hipStream_t s) { add_norm(xt, yin, W.post_norm, d, nullptr, R, P.h, nullptr, s); }});
         }
         {
-            // gate_up only feeds silu * mul: from 65 to 2560 rows it runs unsplit with silu * mul in
-            // the GEMM's epilogue (measured on MI355X at 120 rows: 15.7 us against 13.7 us split in
-            // two plus 4.9 us of silu_mul; the measured plans up to 2560 rows are of the epilogue
-            // kernels); otherwise silu_mul sums the split-K partials itself.  The
+            // gate_up only feeds silu * mul: above 64 rows it runs unsplit with silu * mul in the GEMM's
+            // epilogue (measured on MI355X at 120 rows: 15.7 us against 13.7 us split in two plus 4.9 us
+            // of silu_mul; at 3000 rows the epilogue saves 19 us of silu_mul and 74 MB of big written and
+            // read back); otherwise silu_mul sums the split-K partials itself.  The
             // GEMV rows apply silu * mul in the GEMV's epilogue when the weights are interleaved.
             const Mat m = W.gate_up;
             const bool exact = gemv_rows(m, sr);
             const bool il = gu_il;
-            const int cfu = !exact && m.K % 256 == 0 && R > 64 && R <= 2560 ? gemm_w4_plan(R, m.N, m.K, false, false, 0).cfg : -1;
+            const int cfu = !exact && m.K % 256 == 0 && R > 64 ? gemm_w4_plan(R, m.N, m.K, false, false, 0).cfg : -1;
             if (exact) {
                 const bool fused = il && m.tiled;
                 const GemvPlan gp = gemv_plan(R, m.N, m.K, m.tiled, fused ? 2 : 0, 0);

@@ -941,7 +941,7 @@ int pick_cfg(int M, bool exact) {
 
 // Configuration indices into kCfgs used by the planner: the 64-wide-step 32x32 MFMA tiles (need K a
 // multiple of 256), the same with two k halves per workgroup (K a multiple of 512), and 16x16 tiles.
-constexpr int W21 = 18, W22 = 19, W41 = 20, W31 = 21, W42 = 23, W21h = 24, W41h = 25, W31h = 26;
+constexpr int W21 = 18, W22 = 19, W41 = 20, W31 = 21, W42 = 23, W21h = 24, W41h = 25, W31h = 26, W42h = 27;
 constexpr int T21 = 3, T31 = 4, T41 = 5;  // 16x16 (2,1), (3,1), (4,1)
 // 16x16, loads three steps ahead: (2,1), (3,1), (4,1), (2,2), (3,2)
 constexpr int P21 = 30, P31 = 31, P41 = 32, P22 = 33, P32 = 34;
@@ -952,7 +952,8 @@ constexpr int P21 = 30, P31 = 31, P41 = 32, P22 = 33, P32 = 34;
 // two runs on two boxes averaged; a split plan is charged the consumer's read of its f32 slots (at
 // 5 TB/s); an entry differs from the rules below only where it was at least 3 % faster.  The grid's
 // fill of the 256 CUs decides most entries: the best tile moves with M as the workgroup count
-// crosses multiples of one or two workgroups per CU.
+// crosses multiples of one or two workgroups per CU.  (gate_up from 1729 rows: (4,2), by whole-forward A/B
+// against (4,1): 1800 tokens 7.72 -> 7.54 ms, 2048 8.38 -> 8.19, 2300 9.62 -> 9.53.)
 constexpr int kPlanRows = 37;
 struct MeasuredPlans {
     int N, K;
@@ -1010,8 +1011,8 @@ const MeasuredPlans kMeasured[] = {
          {W41h, 1}, {W21, 1}, {W31, 1}, {W31, 1}, {W21, 1}, {W41, 1}, {W41, 1}, {W31, 1},
          {W31, 1}, {W21, 1}, {W31, 1}, {W31, 1}, {W41, 1}, {W31, 1}, {W31, 1}, {W31, 1},
          {W42, 1}, {W31, 1}, {W31, 1}, {W31, 1}, {W31, 1}, {W31, 1}, {W31, 1}, {W31, 1},
-         {W41, 1}, {W41, 1}, {W41, 1}, {W41, 1}, {W41, 1}, {W41, 1}, {W41, 1}, {W41, 1},
-         {W41, 1}, {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1},
+         {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1},
+         {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1}, {W42, 1},
      }},
     // in_proj
     {8256, 2048,
@@ -1103,7 +1104,17 @@ GemmPlan gemm_w4_plan(int M, int N, int K, bool exact, bool partial_ok, size_t m
         // with k halves where its grid is one round (43.2 us down, 17.6 us o at 1536), else (4,1)
         // (57.9 / 22.3 us at 2048).  The 16x16 (4,2) tiles take 26-50% longer at these sizes.
         const bool one_round = (size_t)((N + 127) / 128) * ((M + 95) / 96) <= 256;
-        if (N >= 10000) p.cfg = M >= 1792 ? W41 : W31;
+        // Above 2560 rows two column tiles per wave: (4,2) reads an A fragment from LDS for two MFMAs, where
+        // (4,1), (3,1) and (2,1) read one for each and need the LDS's whole 128 bytes a clock at the MFMAs'
+        // full rate (counters at 4096 x 12288: MFMAs busy 66% of the clocks for (4,2), 52% for (4,1)).  It pays
+        // once its 128 x 256 tiles are about 1.6 per CU.  us at M = 3000: gate_up 148 against 159 for (4,1),
+        // in_proj 113 / 123 for (3,1), qkv 62 / 72 for (4,1); with fewer tiles and k halves (one workgroup of
+        // 8 waves per CU) down 82.5 / 88 and out_proj 33.3 / 34.7 for (4,1); qkv at 1777 rows, 280 tiles: 51
+        // against 41 for (3,1).
+        const size_t tiles42 = (size_t)((N + 255) / 256) * ((M + 127) / 128);
+        if (M > 2560 && tiles42 >= 400) p.cfg = W42;
+        else if (M > 2560 && halves_ok && tiles42 >= 128 && tiles42 <= 256) p.cfg = W42h;
+        else if (N >= 10000) p.cfg = M >= 1792 ? W41 : W31;
         else if (N >= 7000) p.cfg = W31;
         else if (N >= 4000) p.cfg = W41;
         else p.cfg = halves_ok && one_round ? W31h : W41;

@@ -243,3 +243,19 @@ def test_attention_other_rotary_dims(sdamd, oracle, rd):
     c.run(512, 0)
     err = c.run(40, 512)
     print(f"attention rotary {rd}, L=40 P=512: max |d out| {err:.3g}", flush=True)
+
+
+def test_add_norm_unaligned_y(sdamd, oracle):
+    """y at an address that is a multiple of 2 bytes only: read element by element, bit-identical to the
+    16-byte-aligned call."""
+    rng = np.random.default_rng(8)
+    d, n = 2048, 9
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    y = rng.standard_normal((n, d)).astype(np.float16)
+    w = (1 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    dw, out = dev(w), []
+    for shift in (0, 1):
+        dx, dy, dh = dev(x), dev(np.concatenate([np.zeros(shift, np.float16), y.reshape(-1)])), empty(n * d * 2)
+        sdamd.op_add_norm(dx.data_ptr(), dy.data_ptr() + 2 * shift, dw.data_ptr(), d, None, n, dh.data_ptr(), None)
+        out.append((host(dx, np.float32, (n, d)), host(dh, np.uint16, (n, d))))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
