@@ -107,6 +107,8 @@ bool gemm_w4_has_silu(int cfg);
 // whose rows are interleaved in groups of 16 (interleave_gate_up).
 struct GemvPlan {
     int nct = 1, mt = 1, ks = 1;  // column tiles of 16 per workgroup, row tiles of 16, k splits
+    // plain formats at many rows (k_gemm_fmt): row tiles of 16 per 64-column workgroup, k parts in it
+    int rows = 0, kh = 1;
 };
 GemvPlan gemv_plan(int M, int N, int K, bool tiled, int out, size_t max_part_elems);
 void gemv(const f16* A, const uint32_t* W, const f16* S, const f16* Bi, void* Y, int out, int M, int N, int K, int bits,

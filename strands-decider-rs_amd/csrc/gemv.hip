@@ -2,7 +2,8 @@
 // 550-576), Y[M,N] = A[M,K] f16 . deq(W[N,K])^T with the weights dequantized in f32 and f32
 // accumulation.  It serves the short question suffix (M <= 20, the reference's GEMV rows,
 // src/engine.rs:419-425) and every matrix the tiled kernels do not take: non-default formats
-// (int2/int3, asymmetric, group > 32) and N % 64 != 0 (src/engine.rs:434-442), at any M.
+// (int2/int3, asymmetric, group > 32) and N % 64 != 0 (src/engine.rs:434-442), at any M: k_gemv for few rows,
+// k_gemm_fmt for many.
 //
 // Design (HBM/latency-bound weight streaming):
 //  * v_mfma_f32_16x16x32_f16 with the weights as the row operand (16 output columns) and the
@@ -275,6 +276,207 @@ __global__ __launch_bounds__(256) void k_gemv(const f16* __restrict__ A, const u
     }
 }
 
+// The same product for many rows of the plain formats.  k_gemv dequantizes every weight again for each 32
+// rows and reads A once per 16 columns, which for a 2048 x 2048 matrix at 300 rows is ten dequants and 157 MB
+// of A: 32.8 us.  Here a workgroup takes BM = 16 MT rows x 64 columns (4 waves side by side, 16 columns
+// each), so a weight is dequantized once per BM rows:
+//  * A's step (BM rows x 128 k) goes straight to a ring of 4 LDS stages shared by the waves, the weights and
+//    scales to a ring of 4 register stages, both three steps ahead (the scheme of the int4 kernel with
+//    pipelined loads: 16-byte chunk q of a stage holds row q / 16, k-chunk (q % 16) ^ (row % 16); steps past
+//    the range load zeros, so the waits are exact);
+//  * lane (j, g) dequantizes block g of its column j to the f32 values that k_gemv does, split into the same
+//    f16 hi + lo, in packed steps: 8 codes become 4 f16 pairs 1024 + q by masks; symmetric formats multiply
+//    (q - zero) by the scale in f16 (hi, rounded once) and take the residual with an f16 fma (lo, exact, as the
+//    product is); asymmetric ones take q s + b in f32 (one v_fma_mix_f32 each) and its residual likewise;
+//  * KH = 2: 8 waves, two k parts with their own rings, whose sums meet in LDS (a workgroup's chain of steps,
+//    which a short grid waits for, halves);
+//  * bound by each wave's chain of dequant (int3 asymmetric: about 190 VALU a step), fragment reads (every wave
+//    reads the whole A tile) and MFMAs: 15.5 us for the 2048 x 2048 matrix at 300 rows.  Pinning the dequant
+//    among the MFMAs with scheduling groups made it 21; 128 rows per workgroup 26.
+template <int BITS>
+__device__ __forceinline__ void code_pairs(const typename BlkT<BITS>::T& w, int q, uint32_t (&p)[4]) {
+    constexpr uint32_t EXP = 0x64006400u;  // f16 1024 in both halves: | q gives 1024 + q
+    if constexpr (BITS == 4) {             // element e at bits 4e: x holds 4 of them, the odd ones 16 bits above
+        const uint32_t lo = w[q] & 0xFFFFu, hi = w[q] >> 16, x = lo | (lo << 12), y = hi | (hi << 12);
+        p[0] = and_or(x, 0x000F000Fu, EXP);
+        p[1] = and_or(x >> 8, 0x000F000Fu, EXP);
+        p[2] = and_or(y, 0x000F000Fu, EXP);
+        p[3] = and_or(y >> 8, 0x000F000Fu, EXP);
+    } else {  // element e of the 8 at bits 2e (the low two bits), and for int3 bit e of a byte of w[2]
+        const uint32_t lw = (w[q >> 1] >> (16 * (q & 1))) & 0xFFFFu, x = lw | (lw << 14);
+        uint32_t h = 0;
+        if constexpr (BITS == 3) {
+            const uint32_t hw = (w[2] >> (8 * q)) & 0xFFu;
+            h = (hw << 2) | (hw << 17);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            p[k] = and_or(x >> (4 * k), 0x00030003u, EXP);
+            if constexpr (BITS == 3) p[k] |= (h >> (2 * k)) & 0x00040004u;
+        }
+    }
+}
+
+// a's low or high f16 half times b plus c, in f32 (one rounding)
+__device__ __forceinline__ float mix_lo(uint32_t a, float b, float c) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float mix_hi(uint32_t a, float b, float c) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+template <int BITS, bool ASYM, int MT, bool PARTIAL, int KH>
+__global__ __launch_bounds__(256 * KH) void k_gemm_fmt(const f16* __restrict__ A, const uint32_t* __restrict__ W,
+                                                  const f16* __restrict__ S, const f16* __restrict__ Bi,
+                                                  void* __restrict__ Y, int M, int N, int K, int gdiv, int ks) {
+    typedef typename BlkT<BITS>::T Blk;
+    constexpr int BB = 4 * BITS;             // bytes per quant block
+    constexpr int BM = 16 * MT, BN = 64;
+    constexpr int STAGE = BM * 256;          // bytes of one A stage (128 k of BM rows)
+    constexpr int PER = MT + (ASYM ? 3 : 2);  // vector-memory loads a thread issues per step
+    static_assert(2 * PER <= 63, "vmcnt holds at most 63");
+    static_assert((KH - 1) * MT * 4096 <= KH * STAGE, "the parts' sums fit one stage array");
+    __shared__ __align__(1024) uint8_t As0[KH * STAGE], As1[KH * STAGE], As2[KH * STAGE], As3[KH * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wall = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kh = wall >> 2, wave = wall & 3;  // k part, wave within it
+    uint8_t *const R0 = As0 + kh * STAGE, *const R1 = As1 + kh * STAGE, *const R2 = As2 + kh * STAGE,
+            *const R3 = As3 + kh * STAGE;
+    const int j = lane & 15, g = lane >> 4;
+    int bx, by, bz;
+    xcd_tile(blockIdx.x + (N + BN - 1) / BN * (blockIdx.y + (M + BM - 1) / BM * blockIdx.z), (N + BN - 1) / BN,
+             (M + BM - 1) / BM, ks, bx, by, bz);
+    const int m0 = by * BM, n0 = bx * BN;
+    // K is a multiple of 128; part kh of split bz takes `steps` steps from sb (the last ones perhaps fewer, or
+    // none: their loads are then out of range), `trips` of them run in every part
+    const int KB = K >> 5, SM = K >> 7, SZ = (SM + ks - 1) / ks, trips = (SZ + KH - 1) / KH;
+    const int s1 = min(SM, (bz + 1) * SZ), sb = min(bz * SZ + kh * trips, s1), steps = min(trips, s1 - sb);
+    const int KG = KB / gdiv;
+    const Rsrc ra = make_rsrc(A, (uint32_t)M * K * 2), rw = make_rsrc(W, (uint32_t)N * KB * BB),
+               rs = make_rsrc(S, (uint32_t)N * KG * 2), rb = make_rsrc(ASYM ? Bi : S, (uint32_t)N * KG * 2);
+    uint32_t aoff[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const int q = (i * 4 + wave) * 64 + lane, row = q >> 4, c = (q & 15) ^ (row & 15);
+        aoff[i] = (uint32_t)(min(m0 + row, M - 1) * K + c * 8) * 2u;
+    }
+    const int n = n0 + wave * 16 + j;
+    // fragment read of row tile a, slice s: row 16a + j, k-chunk 4g + s
+    uint32_t foff[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) foff[s] = j * 256 + (((4 * g + s) ^ j) << 4);
+
+    f32x4 acc[MT];
+#pragma unroll
+    for (int a = 0; a < MT; a++) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Blk bw[4];
+    uint32_t bs[4], bb[4];
+    auto issue = [&](int it, uint8_t* dst, int slot) {
+        const bool in = it < steps;
+        const uint32_t ka = in ? (uint32_t)(sb + it) * 256u : OOB;
+        const int b = 4 * (sb + it) + g;
+        const bool ok = in && n < N;
+        const uint32_t wo = ok ? ((uint32_t)n * KB + b) * BB : OOB;
+        const uint32_t so = ok ? ((uint32_t)n * KG + (uint32_t)(b / gdiv)) * 2u : OOB;
+#pragma unroll
+        for (int i = 0; i < MT; i++) buf_lds16(ra, aoff[i], ka, dst + (i * 4 + wave) * 1024);
+        bw[slot] = load_blk<BITS>(rw, wo);
+        bs[slot] = buf_b16(rs, so, 0);
+        if constexpr (ASYM) bb[slot] = buf_b16(rb, so, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto deq = [&](int slot, int q, f16x8& hi, f16x8& lo) {
+        const f16 sc = __builtin_bit_cast(f16, (uint16_t)bs[slot]);
+        uint32_t p[4];
+        code_pairs<BITS>(bw[slot], q, p);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            f16x2 h, l;
+            if constexpr (ASYM) {
+                const float s32 = (float)sc, b32 = (float)__builtin_bit_cast(f16, (uint16_t)bb[slot]);
+                const f16x2 c = __builtin_bit_cast(f16x2, p[k]) - f16x2{(f16)1024.f, (f16)1024.f};
+                const uint32_t cb = __builtin_bit_cast(uint32_t, c);
+                const float v0 = mix_lo(cb, s32, b32), v1 = mix_hi(cb, s32, b32);
+                h = f16x2{(f16)v0, (f16)v1};
+                const uint32_t hb = __builtin_bit_cast(uint32_t, h);
+                const float r0 = mix_lo(hb, -1.0f, v0), r1 = mix_hi(hb, -1.0f, v1);
+                l = f16x2{(f16)r0, (f16)r1};
+            } else {
+                constexpr float Z = 1024.f + (float)(1 << (BITS - 1));
+                const f16x2 c = __builtin_bit_cast(f16x2, p[k]) - f16x2{(f16)Z, (f16)Z}, sc2 = f16x2{sc, sc};
+                h = c * sc2;
+                l = __builtin_elementwise_fma(c, sc2, -h);
+            }
+            hi[2 * k] = h[0], hi[2 * k + 1] = h[1];
+            lo[2 * k] = l[0], lo[2 * k + 1] = l[1];
+        }
+    };
+    auto step = [&](const uint8_t* cur, uint8_t* fill, int slot, int it) {
+        issue(it + 3, fill, (slot + 3) & 3);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            f16x8 hi, lo, af[MT];
+#pragma unroll
+            for (int a = 0; a < MT; a++) af[a] = *reinterpret_cast<const f16x8*>(cur + a * 4096 + foff[s]);
+            deq(slot, s, hi, lo);
+#pragma unroll
+            for (int a = 0; a < MT; a++) acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[a], hi, acc[a], 0, 0, 0);
+#pragma unroll
+            for (int a = 0; a < MT; a++) acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[a], lo, acc[a], 0, 0, 0);
+        }
+        wait_loads<vmcnt_imm(2 * PER)>();  // the loads of steps it + 2, it + 3 may still be in flight
+        bar_noflush();
+    };
+    issue(0, R0, 0);
+    issue(1, R1, 1);
+    issue(2, R2, 2);
+    wait_loads<vmcnt_imm(2 * PER)>();
+    bar_noflush();
+    int it = 0;
+    do {
+        step(R0, R3, 0, it);
+        step(R1, R0, 1, it + 1);
+        step(R2, R1, 2, it + 2);
+        step(R3, R2, 3, it + 3);
+        it += 4;
+    } while (it < trips);
+    wait_loads<vmcnt_imm(0)>();  // the trailing out-of-range loads, before the ring is reused
+    if constexpr (KH > 1) {
+        // the parts' sums, added in k order through the ring: wave w's tile a of part kh at stage a
+        lds_barrier();
+        f32x4* const x = reinterpret_cast<f32x4*>(As0);
+        if (kh)
+#pragma unroll
+            for (int a = 0; a < MT; a++) x[(((kh - 1) * MT + a) * 4 + wave) * 64 + lane] = acc[a];
+        lds_barrier();
+        if (kh) return;
+#pragma unroll
+        for (int p = 1; p < KH; p++)
+#pragma unroll
+            for (int a = 0; a < MT; a++) {
+                const f32x4 v = x[(((p - 1) * MT + a) * 4 + wave) * 64 + lane];
+                acc[a][0] += v[0], acc[a][1] += v[1], acc[a][2] += v[2], acc[a][3] += v[3];
+            }
+    }
+    if (n >= N) return;
+    // acc[a][r] is row m0 + 16a + 4g + r of column n
+#pragma unroll
+    for (int a = 0; a < MT; a++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = m0 + a * 16 + g * 4 + r;
+            if (m >= M) continue;
+            if constexpr (PARTIAL)
+                __builtin_nontemporal_store(acc[a][r], static_cast<float*>(Y) + ((size_t)bz * M + m) * N + n);
+            else
+                static_cast<f16*>(Y)[(size_t)m * N + n] = (f16)acc[a][r];
+        }
+}
+
 typedef void (*GemvFn)(const f16*, const uint32_t*, const f16*, const f16*, void*, int, int, int, int, int);
 
 template <int BITS, bool ASYM, bool TILED, int NCT>
@@ -305,12 +507,44 @@ GemvFn pick_gemv(int bits, bool asym, bool tiled, int nct, int mt, int out) {
     }
 }
 
+// k_gemm_fmt for a plain format
+template <int MT, int KH, bool PARTIAL>
+GemvFn pick_fmt(int bits, bool asym) {
+    switch (bits * 2 + (asym ? 1 : 0)) {
+        case 8: return k_gemm_fmt<4, false, MT, PARTIAL, KH>;
+        case 9: return k_gemm_fmt<4, true, MT, PARTIAL, KH>;
+        case 6: return k_gemm_fmt<3, false, MT, PARTIAL, KH>;
+        case 7: return k_gemm_fmt<3, true, MT, PARTIAL, KH>;
+        case 4: return k_gemm_fmt<2, false, MT, PARTIAL, KH>;
+        case 5: return k_gemm_fmt<2, true, MT, PARTIAL, KH>;
+        default: return nullptr;
+    }
+}
+
 }  // namespace
 
 GemvPlan gemv_plan(int M, int N, int K, bool tiled, int out, size_t max_part_elems) {
     GemvPlan p;
     p.mt = M <= 16 ? 1 : 2;
     const int rb = (M + 16 * p.mt - 1) / (16 * p.mt);
+    // Plain formats whose k_gemv grid (16 columns x 32 rows each) is more than one workgroup per CU: the kernel
+    // that dequantizes a weight once per 32 or 64 rows.  In its grid (64 columns each) two k parts per workgroup
+    // while that is at most one workgroup per CU, 32 rows before 64.  us on MI355X, int3 asymmetric group 64,
+    // k_gemv | 32 rows, 2 parts | 64 rows, 2 parts | 64 rows, 1 part:
+    //   2048 x 2048  64 rows  8.7 | 11.8 | 14.9 | 16.5    96 rows 14.8 | 12.0 | 15.1 | 16.6
+    //               300 rows 32.9 | 20.8 | 15.5 | 17.1   600 rows 64.8 | 31.6 | 30.8 | 27.0   1500: 146 | 63 | 53 | 46
+    //    512 x 2048 200 rows  8.6 | 11.9 | 14.9 | 16.4   300 rows 14.6 | 12.1 | 14.9 | 16.6
+    //   2048 x 6144  64 rows 18.6 | 27.8 | 35.6 | 43.1   300 rows 80.5 | 48.5 | 36.3 | 43.2   1500: 372 | 155 | 121 | 113
+    if (!tiled && out != 2 && K % 128 == 0 && (size_t)((N + 15) / 16) * rb > 256) {
+        const size_t cols = (N + 63) / 64, g2 = cols * ((M + 31) / 32), g4 = cols * ((M + 63) / 64);
+        p.rows = g2 <= 256 ? 2 : 4;
+        p.kh = p.rows == 2 || g4 <= 256 ? 2 : 1;
+        if (out == 1)  // slots for the consumer to add: until the grid covers the chip, parts of at least 4 steps
+            while (p.ks < 8 && (p.rows == 2 ? g2 : g4) * p.ks * 2 <= 256 && K / 128 / (p.ks * 2 * p.kh) >= 4 &&
+                   (size_t)(p.ks * 2) * M * N <= max_part_elems)
+                p.ks *= 2;
+        return p;
+    }
     // f16 outputs own their whole k range; two column tiles per workgroup where that still gives
     // about one workgroup per CU (or more), one otherwise
     p.nct = tiled && (out == 2 || (size_t)((N + 31) / 32) * rb >= 240) ? 2 : 1;
@@ -337,16 +571,25 @@ void gemv(const f16* A, const uint32_t* W, const f16* S, const f16* Bi, void* Y,
     SD_CHECK(p.ks >= 1 && (out == 1 || p.ks == 1), "gemv: only partial outputs split k");
     SD_CHECK((size_t)N * (K / 32) * 4 * bits < 0x80000000u && (size_t)M * K * 2 < 0x80000000u,
              "gemv: operands must be below 2 GiB");
-    const GemvFn f = pick_gemv(bits, asym, tiled, p.nct, p.mt, out);
+    GemvFn f = nullptr;
+    if (p.rows) {
+        SD_CHECK(!tiled && out != 2 && K % 128 == 0 && ((p.rows == 2 && p.kh == 2) || (p.rows == 4 && p.kh <= 2)),
+                 "gemv: no such row tile");
+        if (p.rows == 2) f = out ? pick_fmt<2, 2, true>(bits, asym) : pick_fmt<2, 2, false>(bits, asym);
+        else if (p.kh == 2) f = out ? pick_fmt<4, 2, true>(bits, asym) : pick_fmt<4, 2, false>(bits, asym);
+        else f = out ? pick_fmt<4, 1, true>(bits, asym) : pick_fmt<4, 1, false>(bits, asym);
+    } else {
+        f = pick_gemv(bits, asym, tiled, p.nct, p.mt, out);
+    }
     SD_CHECK(f, "gemv: no kernel for this format and output");
-    const dim3 grid((N + 16 * p.nct - 1) / (16 * p.nct), (M + 16 * p.mt - 1) / (16 * p.mt), p.ks);
+    const dim3 grid = p.rows ? dim3((N + 63) / 64, (M + 16 * p.rows - 1) / (16 * p.rows), p.ks) : dim3((N + 16 * p.nct - 1) / (16 * p.nct), (M + 16 * p.mt - 1) / (16 * p.mt), p.ks);
     const int gdiv = group / 32;
     KernelEvents* ke = kernel_events();
     if (ke && ke->launches == 0) {
-        hipExtLaunchKernelGGL(f, grid, dim3(256), 0, st, ke->start, ke->stop, 0u, A, W, S, Bi, Y, M, N, K, gdiv, p.ks);
+        hipExtLaunchKernelGGL(f, grid, dim3(256 * p.kh), 0, st, ke->start, ke->stop, 0u, A, W, S, Bi, Y, M, N, K, gdiv, p.ks);
         ke->launches++;
     } else {
-        hipLaunchKernelGGL(f, grid, dim3(256), 0, st, A, W, S, Bi, Y, M, N, K, gdiv, p.ks);
+        hipLaunchKernelGGL(f, grid, dim3(256 * p.kh), 0, st, A, W, S, Bi, Y, M, N, K, gdiv, p.ks);
     }
     launched("gemv");
 }
