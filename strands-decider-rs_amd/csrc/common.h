@@ -206,7 +206,7 @@ void gdn_prep(const float* qkvc, const f16* big, const GdnShape& s, const float*
 // only), its old rows from the prefix's history.
 void gdn_scan(const GdnShape& s, int L, const GdnWs& ws, float* state, const uint32_t* lu, int load_default, float* o,
               const Segs& sg, int nseq, hipStream_t st, size_t state_off = 0, f16* hist = nullptr,
-              const f16* big = nullptr, size_t hist_off = 0);
+              const f16* big = nullptr, size_t hist_off = 0, const float* start = nullptr);
 // The same recurrence token by token (the reference's own order), for short inputs: every
 // sequence starts from the prefix state as gdn_scan; with one sequence the final state is written
 // to `state` and hist (nullable) updated afterwards, as gdn_prep + gdn_scan do.

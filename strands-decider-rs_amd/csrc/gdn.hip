@@ -21,9 +21,10 @@
 //    split, in MFMA fragment order, so the scan reads each fragment with one 16-byte load per lane.
 //    The workgroups also perform the reference's hist_update, each on a slice of the channels (the
 //    conv already consumed the old history).
-//  * gdn_scan: one workgroup per (head, 16 value columns), sequential over chunks; the state slice
-//    lives in LDS (transposed, the B operand of every product); 4 waves carry the recurrence and 4
-//    compute the output beside them.
+//  * gdn_scan: one workgroup per (head, 16 value columns), sequential over chunks (or two, that output
+//    every other chunk each); 4 waves carry the recurrence, the state slice f32 in their registers, and 4
+//    compute the output beside them; S and V' pass between them through LDS as the split f16 operands
+//    (transposed, the B operand of every product).
 #include "common.h"
 #include "device.h"
 
@@ -64,6 +65,27 @@ __device__ __forceinline__ void split8(const float* v, f16x8& hi, f16x8& lo) {
     }
 }
 
+// The same for 4 values.
+__device__ __forceinline__ void split4(const f32x4& v, f16x4& hi, f16x4& lo) {
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+        const f16x2 h = f16x2{(f16)v[e], (f16)v[e + 1]};
+        float r0, r1;
+#if defined(__HIP_DEVICE_COMPILE__)
+        const uint32_t hb = __builtin_bit_cast(uint32_t, h);
+        const float v0 = v[e], v1 = v[e + 1];
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hb), "v"(v0));
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hb), "v"(v1));
+#else
+        r0 = v[e] - (float)h[0];
+        r1 = v[e + 1] - (float)h[1];
+#endif
+        hi[e] = h[0];
+        hi[e + 1] = h[1];
+        lo[e] = (f16)r0;
+        lo[e + 1] = (f16)r1;
+    }
+}
 
 // e^x on the hardware exp2 (v_exp_f32, about 1 ulp in f32); x <= 0 here, so the result is in (0, 1].
 __device__ __forceinline__ float fexp(float x) {
@@ -963,28 +985,38 @@ __global__ __launch_bounds__(RT) void k_gdn_recur(const uint32_t* __restrict__ l
 // Sequential over chunks for one head and 16 value columns, in two roles of 4 waves each.  The
 // state role (waves 0-3) carries the recurrence: V' = U - W S, then S <- e^(G_last) S + KgT V';
 // the output role (waves 4-7) computes o = Qg S + Qk V' from the same chunk's S and V'.  Both
-// pass the same two LDS barriers per chunk: after the first, S of chunk c is in St[p]; between
+// pass the same two LDS barriers per chunk: after the first, S of chunk c is in Sh, Sl[p]; between
 // the two, the state role forms W S and V' while the output role forms Qg S; after the second, the
-// state role forms KgT V' and writes chunk c + 1's S into St[p ^ 1] while the output role adds
+// state role forms KgT V' and writes chunk c + 1's S into parity p ^ 1 while the output role adds
 // Qk V' and stores o.  So o's products and operand loads run beside the recurrence instead of on
 // its chain, and each role's CU time goes to its own half of the chunk's operands.  Wave w of a
 // role owns rows 16w..16w+15 of the chunk (and the state role state rows 32w..32w+31 for the
 // update).  The arithmetic of every product is the single-role form's: the same split operands,
 // the same three-chain MFMA sums in the same order.
+// Bound by the CU's vector memory path (112 KB of operands a chunk at about 56 bytes a clock: 2000 of 3000
+// clocks) and the chain of two LDS hand-offs; two workgroups per slice bring the former to 90 KB a chunk
+// (1900 tokens: 1.38 -> 0.97 us a chunk).
 constexpr int SCAN_T = 512;
 __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict__ lu, const uint32_t* __restrict__ seqt,
                                                      const uint32_t* __restrict__ chunkt, float* __restrict__ state,
                                                      int L, int load_default, size_t state_off, float* __restrict__ o,
-                                                     const f16* __restrict__ big, f16* hist, size_t hist_off, GdnShape sh,
-                                                     GdnWs ws) {
+                                                     const f16* __restrict__ big, f16* hist, size_t hist_off,
+                                                     const float* start, GdnShape sh, GdnWs ws) {
     constexpr int DK = 128, DV = 128;
-    constexpr int SP = DK + 4, VP = CH + 4;
-    __shared__ __attribute__((aligned(16))) float St[2][DVS * SP];  // S^T: [column][k], chunk parity p
-    __shared__ __attribute__((aligned(16))) float Vt[DVS * VP];     // V'^T: [column][token]
+    constexpr int SP = DK + 8, VP = CH + 8;  // f16 pitches: 4 banks from row to row
+    // S^T [column][k] by chunk parity and V'^T [column][token], each as the f16 hi and lo parts that the
+    // products take: split once by the wave that computes them (S itself stays f32 in its registers), where
+    // every reader of an f32 copy split all of it again (8 waves x 48 VALU for S, 24 for V', in the chain)
+    __shared__ __attribute__((aligned(16))) f16 Sh[2][DVS * SP], Sl[2][DVS * SP];
+    __shared__ __attribute__((aligned(16))) f16 Vh[DVS * VP], Vl[DVS * VP];
     const int tid = threadIdx.x, lane = tid & 63, w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int role = w8 >> 2, wv = w8 & 3;
     const int fr = lane & 15, fg = lane >> 4;
-    const int h = blockIdx.x, sl = blockIdx.y, H = sh.H, q = blockIdx.z;
+    // A single sequence may come as two workgroups per slice (halves, blockIdx.z): both carry the
+    // recurrence, each outputs every other chunk (the first also keeps the state and history), so a CU
+    // fetches the output's 44 KB of operands for every other chunk only, on CUs that had no work.
+    const int h = blockIdx.x, sl = blockIdx.y, H = sh.H, q = seqt ? (int)blockIdx.z : 0;
+    const int par = seqt ? 0 : (int)blockIdx.z;
     // The lu fields and the sequence's chunk range in one batch of scalar loads, issued before any
     // branch: the pointers are selected first, with `state` standing in for a null table (values
     // then unused).
@@ -992,31 +1024,13 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
     const uint32_t* sp = seqt ? seqt + q : lp;
     const uint32_t lu_nseq = lp[5], lu_load = lp[3], se = *sp;
     const uint8_t* const lu_pre = *reinterpret_cast<const uint8_t* const*>(lp + 8);
-    SGPR_BATCH("s"(lu_nseq), "s"(lu_load), "s"(se), "s"(lu_pre), "s"(hist), "s"(hist_off));
+    SGPR_BATCH("s"(lu_nseq), "s"(lu_load), "s"(se), "s"(lu_pre), "s"(hist), "s"(hist_off), "s"(start));
     if (seqt && q >= (int)lu_nseq) return;  // the grid is sized for the most sequences
     const int c0 = sl * DVS;
     const bool load = lu ? lu_load != 0u : load_default != 0;
     const uint8_t* pre = lu ? lu_pre : nullptr;
     float* Sg = state + (size_t)h * DK * DV;  // the live state (written back by a single sequence)
-    const float* S0 = (pre ? reinterpret_cast<const float*>(pre + state_off) : state) + (size_t)h * DK * DV;
-    {
-        // The slice through a buffer resource, every load issued before the first LDS store (a load
-        // under a branch, or a flat one, would be waited for before the next is issued); a fresh
-        // state gets an empty resource, whose loads return 0 without touching memory.
-        static_assert(DK * DVS % SCAN_T == 0, "whole passes of the workgroup");
-        const Rsrc rs = make_rsrc(S0, load ? (uint32_t)(DK * DV * 4) : 0u);
-        float sv[DK * DVS / SCAN_T];
-#pragma unroll
-        for (int i = 0; i < DK * DVS / SCAN_T; i++) {
-            const int e = tid + SCAN_T * i, k = e / DVS, cc = e % DVS;
-            sv[i] = __builtin_bit_cast(float, buf_b32(rs, (uint32_t)((k * DV + c0 + cc) * 4), 0u));
-        }
-#pragma unroll
-        for (int i = 0; i < DK * DVS / SCAN_T; i++) {
-            const int e = tid + SCAN_T * i, k = e / DVS, cc = e % DVS;
-            St[0][cc * SP + k] = sv[i];
-        }
-    }
+    const float* S0 = (pre ? reinterpret_cast<const float*>(pre + state_off) : start ? start : state) + (size_t)h * DK * DV;
     // the reference's hist_update (src/kernels.rs:173-190): the last 3 rows of (the prefix's history
     // ++ this forward's rows) become the live history, each workgroup on a slice of the channels;
     // here, after the prep that read the old history for its conv.  This thread's channel lo + tid
@@ -1025,7 +1039,7 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
     const int hlo = (blockIdx.y * H + h) * hper, hhi = min(hC, hlo + hper);
     const f16* hold = pre ? reinterpret_cast<const f16*>(pre + hist_off) : hist;
     f16 hv[3] = {};
-    if (hist && hlo + tid < hhi) {
+    if (hist && par == 0 && hlo + tid < hhi) {
 #pragma unroll
         for (int r = 0; r < 3; r++) {
             const int src = L - 3 + r;
@@ -1069,21 +1083,17 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
         hi = __builtin_bit_cast(f16x8, buf_b128(rws, vf, so));
         lo = __builtin_bit_cast(f16x8, buf_b128(rws, vf, so + 1024u));
     };
-    // S^T slice of k step s for this lane (column fr, k = 32 s + 8 fg ..), from St[p]
-    auto s_slice = [&](int p, int s, float* v8) {
-        const float* spp = &St[p][fr * SP + s * 32 + fg * 8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) v8[u] = spp[u];
+    // S^T fragments of k step s for this lane (column fr, k = 32 s + 8 fg ..), from parity p
+    auto s_frag = [&](int p, int s, f16x8& hi, f16x8& lo) {
+        hi = *reinterpret_cast<const f16x8*>(&Sh[p][fr * SP + s * 32 + fg * 8]);
+        lo = *reinterpret_cast<const f16x8*>(&Sl[p][fr * SP + s * 32 + fg * 8]);
     };
     // V'^T fragments (B operand) of the chunk, both k steps
     auto v_frags = [&](f16x8 (&vh)[2], f16x8 (&vl)[2]) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            float v8[8];
-            const float* vp = &Vt[fr * VP + s * 32 + fg * 8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v8[u] = vp[u];
-            split8(v8, vh[s], vl[s]);
+            vh[s] = *reinterpret_cast<const f16x8*>(&Vh[fr * VP + s * 32 + fg * 8]);
+            vl[s] = *reinterpret_cast<const f16x8*>(&Vl[fr * VP + s * 32 + fg * 8]);
         }
     };
     const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
@@ -1093,6 +1103,27 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
         WS set0, set1;
         f16x8 kh[2][2], kl[2][2];
         float gl = 0.f;
+        // the state: rows (2 wv + q2) 16 + 4 fg + r of column c0 + fr.  Its loads go through a buffer
+        // resource (a flat load would also count as an LDS operation); a fresh state gets an empty one,
+        // whose loads return 0 without touching memory.
+        f32x4 S[2];
+        const Rsrc rs0 = make_rsrc(S0, load ? (uint32_t)(DK * DV * 4) : 0u);
+        const uint32_t vs = (uint32_t)((fg * 4 * DV + c0 + fr) * 4);
+#pragma unroll
+        for (int q2 = 0; q2 < 2; q2++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                S[q2][r] = __builtin_bit_cast(float, buf_b32(rs0, vs, (uint32_t)(((wv * 2 + q2) * 16 + r) * DV * 4)));
+        auto put_s = [&](int p) {  // S's hi and lo parts into parity p
+#pragma unroll
+            for (int q2 = 0; q2 < 2; q2++) {
+                f16x4 hi, lo;
+                split4(S[q2], hi, lo);
+                const int so = fr * SP + (wv * 2 + q2) * 16 + fg * 4;
+                *reinterpret_cast<f16x4*>(&Sh[p][so]) = hi;
+                *reinterpret_cast<f16x4*>(&Sl[p][so]) = lo;
+            }
+        };
         auto load_w_step = [&](WS& d, int cc, int s) {
             const uint32_t vf = cc < cend ? vfrag : OOB;
             frag(slot_of(cc) * (uint32_t)(WF_H * 2), 4, wv, s, d.wh[s], d.wl[s], vf);
@@ -1113,29 +1144,29 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
         };
         auto chunk = [&](int cc, int p, const WS& cur, WS& nxt) {
             load_u(nxt, cc + 1);
-            lds_barrier();  // St[p] holds this chunk's starting state; Vt is free
+            lds_barrier();  // parity p holds this chunk's starting state; V' is free
             f32x4 av[3] = {z4, z4, z4};
-            // k step s: its S slice (read from LDS during step s - 1), then the next chunk's W loads
-            // of step s, each step a scheduling region of its own so that those loads are issued
-            // in four groups
-            float sn[8];
-            s_slice(p, 0, sn);
+            // k step s: its S fragments (all read at once), then the next chunk's W loads of step s, each
+            // step a scheduling region of its own so that those loads are issued in four groups
+            f16x8 sh8[4], sl8[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) s_frag(p, s, sh8[s], sl8[s]);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                float s8[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) s8[u] = sn[u];
-                if (s < 3) s_slice(p, s + 1, sn);
                 load_w_step(nxt, cc + 1, s);
-                f16x8 sh8, sl8;
-                split8(s8, sh8, sl8);
-                mma3s(cur.wh[s], cur.wl[s], sh8, sl8, av);
+                mma3s(cur.wh[s], cur.wl[s], sh8[s], sl8[s], av);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            // rows wv * 16 + fg * 4 .. + 3 of column fr: one 16-byte store (conflict-free at this pitch)
-            *reinterpret_cast<float4*>(&Vt[fr * VP + wv * 16 + fg * 4]) =
-                float4{cur.ur[0] - (av[0][0] + av[1][0] + av[2][0]), cur.ur[1] - (av[0][1] + av[1][1] + av[2][1]),
-                       cur.ur[2] - (av[0][2] + av[1][2] + av[2][2]), cur.ur[3] - (av[0][3] + av[1][3] + av[2][3])};
+            // rows wv * 16 + fg * 4 .. + 3 of column fr: two 8-byte stores
+            {
+                f32x4 v;
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = cur.ur[r] - (av[0][r] + av[1][r] + av[2][r]);
+                f16x4 hi, lo;
+                split4(v, hi, lo);
+                *reinterpret_cast<f16x4*>(&Vh[fr * VP + wv * 16 + fg * 4]) = hi;
+                *reinterpret_cast<f16x4*>(&Vl[fr * VP + wv * 16 + fg * 4]) = lo;
+            }
             lds_barrier();  // V' complete
             f16x8 vh[2], vl[2];
             v_frags(vh, vl);
@@ -1152,16 +1183,10 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int q2 = 0; q2 < 2; q2++) {
-                // state rows k0 .. k0 + 3 of column fr: one 16-byte read of S_c and one write of S_c+1
-                const int so = fr * SP + (wv * 2 + q2) * 16 + fg * 4;
-                const float4 s4 = *reinterpret_cast<const float4*>(&St[p][so]);
-                *reinterpret_cast<float4*>(&St[p ^ 1][so]) =
-                    float4{g_c * s4.x + (as[q2][0][0] + as[q2][1][0] + as[q2][2][0]),
-                           g_c * s4.y + (as[q2][0][1] + as[q2][1][1] + as[q2][2][1]),
-                           g_c * s4.z + (as[q2][0][2] + as[q2][1][2] + as[q2][2][2]),
-                           g_c * s4.w + (as[q2][0][3] + as[q2][1][3] + as[q2][2][3])};
-            }
+            for (int q2 = 0; q2 < 2; q2++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) S[q2][r] = g_c * S[q2][r] + (as[q2][0][r] + as[q2][1][r] + as[q2][2][r]);
+            put_s(p ^ 1);
         };
 #pragma unroll
         for (int s = 0; s < 4; s++) load_w_step(set0, cfirst, s);
@@ -1169,11 +1194,18 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
         load_gl(cfirst);
         load_kg(cfirst, 0);
         load_kg(cfirst, 1);
+        put_s(0);
         for (; c + 1 < cend; c += 2) {  // no branch inside the loop body
             chunk(c, 0, set0, set1);
             chunk(c + 1, 1, set1, set0);
         }
         if (c < cend) chunk(c, 0, set0, set1);
+        if (!seqt && par == 0) {  // several sequences: their final states are not kept
+#pragma unroll
+            for (int q2 = 0; q2 < 2; q2++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) Sg[((wv * 2 + q2) * 16 + fg * 4 + r) * DV + c0 + fr] = S[q2][r];
+        }
     } else {
         // ---- output role: o = Qg S + Qk V'
         QS set0, set1;
@@ -1185,29 +1217,26 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
         auto load_qk = [&](int cc) {
             const uint32_t vf = cc < cend ? vfrag : OOB, slot = slot_of(cc);
 #pragma unroll
-            for (int s = 0; s < 2; s++) frag(o_qk + slot * (uint32_t)(QKF_H * 2), 2, wv, s, qkh[s], qkl[s], vf);
+            for (int s = 0; s < 2; s++)  // row tiles 0 and 1 lie wholly above k step 1's diagonal: zeros
+                frag(o_qk + slot * (uint32_t)(QKF_H * 2), 2, wv, s, qkh[s], qkl[s], s && wv < 2 ? OOB : vf);
         };
         // o rows t0 + wv*16 + fg*4 + r (r < 4), column h*DV + c0 + fr; rows past the chunk get an
         // out-of-range offset and are not written
         const Rsrc ro = make_rsrc(o, (uint32_t)L * sh.H * DV * 4);
         const uint32_t vo = (uint32_t)((fg * 4 * sh.H * DV + fr) * 4);
-        auto chunk = [&](int cc, int p, const QS& cur, QS& nxt) {
+        // chunk cc, loading the operands of chunk cn behind its own
+        auto chunk = [&](int cc, int p, int cn, const QS& cur, QS& nxt) {
             const int t0 = chunkt ? (int)(chunkt[cc] & 0xFFFFu) : cc * CH;
             const int Lc = chunkt ? (int)(chunkt[cc] >> 16) : min(CH, L - cc * CH);
-            lds_barrier();  // St[p] holds this chunk's starting state
+            lds_barrier();  // parity p holds this chunk's starting state
             f32x4 ao[3] = {z4, z4, z4};
-            float sn[8];
-            s_slice(p, 0, sn);
+            f16x8 sh8[4], sl8[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) s_frag(p, s, sh8[s], sl8[s]);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                float s8[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) s8[u] = sn[u];
-                if (s < 3) s_slice(p, s + 1, sn);
-                load_q_step(nxt, cc + 1, s);
-                f16x8 sh8, sl8;
-                split8(s8, sh8, sl8);
-                mma3s(cur.qh[s], cur.ql[s], sh8, sl8, ao);
+                load_q_step(nxt, cn, s);
+                mma3s(cur.qh[s], cur.ql[s], sh8[s], sl8[s], ao);
                 __builtin_amdgcn_sched_barrier(0);
             }
             lds_barrier();  // V' complete
@@ -1215,7 +1244,7 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
             v_frags(vh, vl);
 #pragma unroll
             for (int s = 0; s < 2; s++) mma3s(qkh[s], qkl[s], vh[s], vl[s], ao);
-            load_qk(cc + 1);  // Qk is consumed
+            load_qk(cn);  // Qk is consumed
             __builtin_amdgcn_sched_barrier(0);
             const uint32_t so = (uint32_t)(((t0 + wv * 16) * sh.H * DV + h * DV + c0) * 4);
 #pragma unroll
@@ -1225,23 +1254,39 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
                          __builtin_bit_cast(uint32_t, ao[0][r] + ao[1][r] + ao[2][r]));
             }
         };
+        const bool halves = !seqt && gridDim.z > 1;
+        const int first = cfirst + par, hop = halves ? 2 : 1;
 #pragma unroll
-        for (int s = 0; s < 4; s++) load_q_step(set0, cfirst, s);
-        load_qk(cfirst);
-        for (; c + 1 < cend; c += 2) {
-            chunk(c, 0, set0, set1);
-            chunk(c + 1, 1, set1, set0);
+        for (int s = 0; s < 4; s++) load_q_step(set0, first, s);
+        load_qk(first);
+        auto skip = [&]() {  // the other half's chunk: the barriers alone
+            lds_barrier();
+            lds_barrier();
+        };
+        if (halves) {
+            if (par) {
+                skip();
+                c++;
+            }
+            for (; c + 2 < cend; c += 4) {  // chunks c and c + 2, of one parity
+                chunk(c, par, c + hop, set0, set1);
+                skip();
+                chunk(c + 2, par, c + 2 + hop, set1, set0);
+                if (c + 3 < cend) skip();
+            }
+            if (c < cend) {
+                chunk(c, par, c + hop, set0, set1);
+                if (c + 1 < cend) skip();
+            }
+        } else {
+            for (; c + 1 < cend; c += 2) {
+                chunk(c, 0, c + 1, set0, set1);
+                chunk(c + 1, 1, c + 2, set1, set0);
+            }
+            if (c < cend) chunk(c, 0, c + 1, set0, set1);
         }
-        if (c < cend) chunk(c, 0, set0, set1);
     }
-    if (seqt) return;  // several sequences: their final states are not kept
-    __syncthreads();
-    const int pf = (cend - cfirst) & 1;  // the buffer holding the final state
-    for (int e = tid; e < DK * DVS; e += SCAN_T) {
-        const int k = e / DVS, cc = e % DVS;
-        Sg[k * DV + c0 + cc] = St[pf][cc * SP + k];
-    }
-    if (hist) {
+    if (hist && par == 0) {
         if (hlo + tid < hhi) {
 #pragma unroll
             for (int r = 0; r < 3; r++) hist[(size_t)r * hC + hlo + tid] = hv[r];
@@ -1361,13 +1406,20 @@ void gdn_prep(const float* qkvc, const f16* big, const GdnShape& s, const float*
 }
 
 void gdn_scan(const GdnShape& s, int L, const GdnWs& ws, float* state, const uint32_t* lu, int load_default, float* o,
-              const Segs& sg, int nseq, hipStream_t st, size_t state_off, f16* hist, const f16* big, size_t hist_off) {
+              const Segs& sg, int nseq, hipStream_t st, size_t state_off, f16* hist, const f16* big, size_t hist_off,
+              const float* start) {
     SD_CHECK(s.DK == 128 && s.DV == 128, "gated delta net: only 128-wide key/value heads are supported");
     SD_CHECK(!sg.seq || (lu && sg.chunk), "gdn_scan: several sequences need lu and the chunk table");
     SD_CHECK(!hist || (!sg.seq && big), "gdn_scan: the history update needs one sequence and big");
-    if (!sg.seq) nseq = 1;
+    // One sequence of several chunks on a grid that leaves half the CUs idle runs as two workgroups per slice
+    // (prep + scan on MI355X, one against two: 512 tokens 30.2 -> 29.1 us, 1024 38.5 -> 34.9, 1900 66.7 -> 60.0,
+    // 3000 103 -> 93).  Not where the state it starts from is the one it writes: the first may have written
+    // it before the second starts.  (With lu a single sequence starts from a snapshot or from nothing.)
+    const bool in_place = !lu && load_default && !start;
+    const int halves = !in_place && L > CH && s.H * (s.DV / DVS) * 2 <= 256 ? 2 : 1;
+    if (!sg.seq) nseq = halves;
     hipLaunchKernelGGL(k_gdn_scan, dim3(s.H, s.DV / DVS, nseq), dim3(SCAN_T), 0, st, lu, sg.seq, sg.chunk, state, L,
-                       load_default, state_off, o, big, hist, hist_off, s, ws);
+                       load_default, state_off, o, big, hist, hist_off, start, s, ws);
     launched("gdn_scan");
 }
 

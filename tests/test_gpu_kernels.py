@@ -127,6 +127,7 @@ def oracle_gdn(oracle, qkv, big, stride, nA, db, L, H, state0, load):
     import ctypes
     st = state0.copy()
     o = np.empty((L, H * 128), np.float32)
+    import ctypes
     I = ctypes.c_int
     oracle.lib().or_gdn(oracle.P(qkv), oracle.P(big.view(np.uint16)), I(stride), I(0), I(H), oracle.P(nA),
                         oracle.P(db), I(L), I(H), I(128), I(128), oracle.P(st), I(int(load)), oracle.P(o))
@@ -317,3 +318,31 @@ def test_gate_up_silu(sdamd, synth, oracle, M, exact, cfg):
     tol = 2.01 * f16_ulp(want) + np.abs(dsilu * u) * dg + np.abs(g * sig) * du + 1e-6
     err = np.abs(got - want)
     assert (err <= tol).all(), f"{(err > tol).sum()} beyond tolerance; max err {err.max()}"
+
+
+@pytest.mark.parametrize("L,load", [(65, False), (128, True), (193, False), (320, False), (1025, True), (1088, True)])
+def test_gdn_halves_match_one_workgroup_per_slice(sdamd, oracle, L, load):
+    """Chunk counts 2 (ragged and whole), 4, 5 and 17 (ragged and whole) of a single sequence, whose scan runs as two
+    workgroups per slice (output of every other chunk each), from nothing, from a state in place (one workgroup)
+    and from a copy of it (from 1024 tokens on), against the oracle's sequential rule: 2e-4, as the other
+    delta-rule tests."""
+    rng = np.random.default_rng(L)
+    H, dk, dv = 16, 128, 128
+    C = 2 * H * dk + H * dv
+    qkv = rng.standard_normal((L, C)).astype(np.float32)
+    big = rng.standard_normal((L, 2 * H)).astype(np.float16)
+    nA = (-rng.uniform(0.02, 2.0, H)).astype(np.float32)
+    dtb = np.zeros(H, np.float32)
+    S0 = (0.3 * rng.standard_normal((H, dk, dv))).astype(np.float32) if load else np.zeros((H, dk, dv), np.float32)
+    dq, db, dn, dd, ds = dev(qkv), dev(big), dev(nA), dev(dtb), dev(S0)
+    do_ = torch.zeros(L * H * dv * 4, dtype=torch.uint8, device="cuda")
+    sdamd.op_gdn(dq.data_ptr(), db.data_ptr(), 2 * H, 0, H, dn.data_ptr(), dd.data_ptr(), L, H, dk, dv, ds.data_ptr(),
+                 load, do_.data_ptr())
+    torch.cuda.synchronize()
+    want, S = np.empty((L, H * dv), np.float32), S0.copy()
+    import ctypes
+    I = ctypes.c_int
+    oracle.lib().or_gdn(oracle.P(qkv), oracle.P(big.view(np.uint16)), I(2 * H), I(0), I(H), oracle.P(nA), oracle.P(dtb),
+                        I(L), I(H), I(dk), I(dv), oracle.P(S), I(int(load)), oracle.P(want))
+    assert np.abs(host(do_, np.float32, (L, H * dv)) - want).max() < 2e-4
+    assert np.abs(host(ds, np.float32, (H, dk, dv)) - S).max() < 2e-4
