@@ -190,6 +190,11 @@ constexpr int PREP_T = 512;  // k_gdn_prep threads: 8 waves
 // CONV: q, k and v are the causal conv + SiLU of big's rows, computed here (the reference's conv,
 // src/kernels.rs:152-170: rows before a sequence's start from the history, the prefix snapshot's when
 // lu names one); otherwise they are read from qkvc.
+// A workgroup is a chain of short phases, and a long input's many rounds also write 140 KB of operands a slot
+// (at 3000 rows two fifths to a half of the time at a copy's rate).  What lies above the diagonal of T, Qk and
+// Kn Kn^T is neither computed nor written where a whole tile of it does: 6 of 16 tiles of the products, 4 of 16 of
+// T's splits, 2 of 8 of Qk's fragments.  Whole op, with that work -> without, over two runs each: 17.1 -> 16.8 us at 65 rows,
+// 28.9 -> 28.6 at 512, 60.1 -> 59.3 at 1900.
 template <bool CONV>
 // Kernel arguments: the pointers and ints first, the structs last (the first 16 dwords are preloaded
 // into SGPRs, up to the first struct; the prologue needs the tables and big before anything else).
@@ -449,16 +454,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(PREP_T, PREP_T), amdgpu_wa
     }
 
     // ---- phase 1: Kn Kn^T (T side) or Qn Kn^T (q side); wave w computes row tile w % 4 x column
-    // tiles 2 (w / 4), 2 (w / 4) + 1
+    // tiles 2 (w / 4), 2 (w / 4) + 1, those that reach the diagonal (the others are masked whole)
     {
-        const int wr = wv & 3, tc = 2 * (wv >> 2);
+        const int wu = __builtin_amdgcn_readfirstlane(wv), wr = wu & 3, tc = 2 * (wu >> 2);
         f32x4 acc[2];
 #pragma unroll
         for (int t = 0; t < 2; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         const f16* Ah = qside ? Qh : Kh;
         const f16* Al = qside ? Ql : Kl;
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
+        for (int s = 0; s < 4 && tc <= wr; s++) {
             const int ar = (wr * 16 + fr) * RP + s * 32 + fg * 8;
             const f16x8 ah = *reinterpret_cast<const f16x8*>(&Ah[ar]), al = *reinterpret_cast<const f16x8*>(&Al[ar]);
 #pragma unroll
@@ -490,8 +495,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(PREP_T, PREP_T), amdgpu_wa
             }
         lds_barrier();
         if (qside) {
-            // Qk as A fragments: 4 row tiles x 2 k steps x 64 lanes, one per thread
-            const int ln = tid & 63, st = (tid >> 6) & 1, rt = tid >> 7;
+            // Qk as A fragments: 4 row tiles x 2 k steps x 64 lanes, one per thread; k step 1 of row tiles 0 and 1
+            // lies wholly above the diagonal and is not fetched by the scan
+            const int ln = tid & 63, st = wu & 1, rt = wu >> 1;
+            if (st && rt < 2) return;
             const float* src = &Qs[(rt * 16 + (ln & 15)) * FP + st * 32 + (ln >> 4) * 8];
             float v8[8];
 #pragma unroll
@@ -573,7 +580,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(PREP_T, PREP_T), amdgpu_wa
         for (int rt = 0; rt < 4; rt++) {
             aw[rt] = au[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s = 0; s < 2; s++) {
+            for (int s = 0; s <= rt / 2; s++) {  // T is lower triangular: rows 0 .. 31 take no token past 31
                 const float* tp = &Ts[(rt * 16 + fr) * FP + s * 32 + fg * 8];
                 const float4 t0v = *reinterpret_cast<const float4*>(tp), t1v = *reinterpret_cast<const float4*>(tp + 4);
                 const float t8[8] = {t0v.x, t0v.y, t0v.z, t0v.w, t1v.x, t1v.y, t1v.z, t1v.w};
