@@ -535,7 +535,12 @@ GemvPlan gemv_plan(int M, int N, int K, bool tiled, int out, size_t max_part_ele
     //               300 rows 32.9 | 20.8 | 15.5 | 17.1   600 rows 64.8 | 31.6 | 30.8 | 27.0   1500: 146 | 63 | 53 | 46
     //    512 x 2048 200 rows  8.6 | 11.9 | 14.9 | 16.4   300 rows 14.6 | 12.1 | 14.9 | 16.6
     //   2048 x 6144  64 rows 18.6 | 27.8 | 35.6 | 43.1   300 rows 80.5 | 48.5 | 36.3 | 43.2   1500: 372 | 155 | 121 | 113
-    if (!tiled && out != 2 && K % 128 == 0 && (size_t)((N + 15) / 16) * rb > 256) {
+    // Up to 16 rows most of its 32 are padding, for k_gemv half of 32: more than two workgroups per CU, and 8 rows.
+    // Six formats of int2 to int4, K = 2048, k_gemv's time over this kernel's (least, most):
+    //   N = 5120: 8 rows 0.76, 0.99  16 rows 0.87, 1.11  17 rows 1.02, 1.36  33 rows 1.32, 1.71
+    //   N = 8256: 4 rows 0.96, 1.29   8 rows 1.04, 1.34  17 rows 1.44, 1.85;  N = 12288: 4 rows 0.99, 1.32  8 rows 1.06, 1.35
+    const size_t blocks = (size_t)((N + 15) / 16) * rb;
+    if (!tiled && out != 2 && K % 128 == 0 && blocks > 256 && (M > 16 || (M >= 8 && blocks > 512))) {
         const size_t cols = (N + 63) / 64, g2 = cols * ((M + 31) / 32), g4 = cols * ((M + 63) / 64);
         p.rows = g2 <= 256 ? 2 : 4;
         p.kh = p.rows == 2 || g4 <= 256 ? 2 : 1;

@@ -42,6 +42,13 @@ def test_many_rows(sdamd, oracle, M, N, K, bits, group, asym):
     assert (err <= 1.01 * f16_ulp(want) + 2e-5).all(), f"max err {err.max()}"
 
 
+@pytest.mark.parametrize("M,N", [(7, 8256), (8, 8192), (8, 8256), (16, 5120), (16, 8256), (17, 4096), (17, 4112)])
+def test_both_sides_of_the_line_at_few_rows(sdamd, oracle, M, N):
+    """Up to 16 rows the kernel runs from 8 rows and 513 blocks of 16 columns on, above from 257 on; the GEMV
+    takes the others."""
+    test_many_rows(sdamd, oracle, M, N, 256, 3, 64, True)
+
+
 def test_rows_past_the_last_are_not_written(sdamd):
     """The output ends at row M (a tile holds 32 or 64)."""
     M, N, K = 65, 2048, 256
