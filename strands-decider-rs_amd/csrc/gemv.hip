@@ -566,7 +566,16 @@ GemvPlan gemv_plan(int M, int N, int K, bool tiled, int out, size_t max_part_ele
 }
 
 void gemv(const f16* A, const uint32_t* W, const f16* S, const f16* Bi, void* Y, int out, int M, int N, int K, int bits,
-          int group, bool asym, bool tiled, const GemvPlan& p, hipStream_t st) {
+          int group, bool asym, bool tiled, const GemvPlan& plan, hipStream_t st) {
+    GemvPlan p = plan;
+    if (p.rows && reinterpret_cast<uintptr_t>(A) % 16) {
+        // k_gemm_fmt moves A's 16-byte pieces straight to LDS: an A that does not start on one keeps k_gemv,
+        // which loads it to registers, with the same k splits
+        p.nct = 1;
+        p.mt = M <= 16 ? 1 : 2;
+        p.rows = 0;
+        p.kh = 1;
+    }
     SD_CHECK(M >= 1 && N >= 1 && K >= 32 && K % 32 == 0, "gemv: need M, N >= 1 and K a multiple of 32");
     SD_CHECK(bits == 2 || bits == 3 || bits == 4, "gemv: weights must be int2, int3 or int4");
     SD_CHECK(group >= 32 && group % 32 == 0 && K % group == 0, "gemv: the group must be a multiple of 32 dividing K");

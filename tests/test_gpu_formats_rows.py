@@ -49,6 +49,26 @@ def test_both_sides_of_the_line_at_few_rows(sdamd, oracle, M, N):
     test_many_rows(sdamd, oracle, M, N, 256, 3, 64, True)
 
 
+def test_rows_that_start_between_16_byte_pieces(sdamd):
+    """A at 8 bytes past a piece (the GEMV takes it): the aligned call's result, but for the f32 summation order."""
+    from conftest import f16_ulp
+    M, N, K = 80, 2048, 512
+    rng = np.random.default_rng(3)
+    A = rng.standard_normal((M, K)).astype(np.float16)
+    W = gcases.pack_codes(rng.integers(0, 8, size=(N, K), dtype=np.uint32), 3)
+    S, B = (rng.uniform(-0.05, 0.05, size=N * K // 64).astype(np.float16) for _ in range(2))
+    dA, dW, dS, dB = dev(A), dev(W), dev(S), dev(B)
+    dU = torch.zeros(M * K * 2 + 16, dtype=torch.uint8, device="cuda")
+    dU[8:8 + M * K * 2] = dA
+    got = []
+    for a in (dA.data_ptr(), dU.data_ptr() + 8):
+        y = torch.zeros(M * N * 2, dtype=torch.uint8, device="cuda")
+        sdamd.op_matmul_fmt(a, dW.data_ptr(), dS.data_ptr(), dB.data_ptr(), y.data_ptr(), M, N, K, 3, 64, True)
+        torch.cuda.synchronize()
+        got.append(y.cpu().numpy().view(np.float16).astype(np.float32))
+    assert (np.abs(got[0] - got[1]) <= 1.01 * f16_ulp(got[0]) + 2e-5).all()
+
+
 def test_rows_past_the_last_are_not_written(sdamd):
     """The output ends at row M (a tile holds 32 or 64)."""
     M, N, K = 65, 2048, 256
