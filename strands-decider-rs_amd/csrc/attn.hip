@@ -1041,7 +1041,10 @@ void attention_split(const f16* Q, const f16* Kc, const f16* Vc, const f16* big,
     float* pacc = ws;
     float* pml = ws + (size_t)p.ks * L * s.HQ * s.HD;
     const int G = s.HQ / s.HK;
-    if (p.rows) {
+    // k_attn_rows moves the cache's 16-byte pieces straight to LDS: a cache that does not start on one keeps
+    // k_attn, which loads them to registers (with the same key splits)
+    const bool pieces = (reinterpret_cast<uintptr_t>(Kc) | reinterpret_cast<uintptr_t>(Vc)) % 16 == 0;
+    if (p.rows && pieces) {
         SD_CHECK(G <= 32 && (G & (G - 1)) == 0, "attention: a tile of 32 rows takes a power of two of query heads");
         const auto f = Q ? k_attn_rows<256, 0> : k_attn_rows<256, 64>;
         hipLaunchKernelGGL(f, dim3(s.HK, (L * G + 31) / 32, p.ks), dim3(256), 0, st, Q, Kc, Vc, lu, L, s.HQ, s.HK, s.stride,

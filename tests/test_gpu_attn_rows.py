@@ -18,7 +18,7 @@ def dev(a):
     return torch.from_numpy(a.view(np.uint8).reshape(-1).copy()).cuda()
 
 
-def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0):
+def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0):
     """P prefix rows straight in the cache, then L rows; out within 2 f16 ulp + 1e-3 of the oracle (scores,
     softmax and P V in f32 against the oracle's f64 softmax: the bound of the other attention tests)."""
     from conftest import f16_ulp
@@ -33,6 +33,10 @@ def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0):
     oV[:, :P] = rng.standard_normal((hk, P, HD)).astype(np.float16).view(np.uint16)
     dK = dev(oK.reshape(hk, CTX // 32, 32, HD // 32, 32).transpose(0, 1, 3, 2, 4))
     dV = dev(oV.reshape(hk, CTX // 32, 32, HD).transpose(0, 1, 3, 2))
+    if shift:  # the cache starts `shift` bytes past a 16-byte piece
+        pad = torch.zeros(shift, dtype=torch.uint8, device="cuda")
+        dK, dV = (torch.cat([pad, t])[shift:] for t in (dK, dV))
+        assert dK.data_ptr() % 16 == shift and dV.data_ptr() % 16 == shift
     dbig, dqw, dkw, drope = dev(big), dev(qw), dev(kw), dev(rope)
     dQ = torch.zeros(hq * L * HD * 2, dtype=torch.uint8, device="cuda")
     dout = torch.zeros(L * hq * HD * 2, dtype=torch.uint8, device="cuda")
@@ -65,6 +69,12 @@ def test_rows_kernel_edges(sdamd, oracle, L, P):
 def test_rows_kernel_groups(sdamd, oracle, hq, hk):
     """1, 2, 8 and 16 query heads per kv head (32, 16, 4 and 2 queries per tile); 3 take the other kernel."""
     check(sdamd, oracle, 7 * hq + hk, hq, hk, 141, 50)
+
+
+@pytest.mark.parametrize("L,P", [(160, 0), (160, 70), (300, 33)])
+def test_cache_that_starts_between_16_byte_pieces(sdamd, oracle, L, P):
+    """The other kernel takes it, with and without key splits."""
+    check(sdamd, oracle, 3 * L + P, 8, 2, L, P, shift=8)
 
 
 def test_rows_kernel_reads_prepared_queries(sdamd, oracle):
