@@ -1003,8 +1003,13 @@ __global__ __launch_bounds__(RT) void k_gdn_recur(const uint32_t* __restrict__ l
 // Bound by the CU's vector memory path (112 KB of operands a chunk at about 56 bytes a clock: 2000 of 3000
 // clocks) and the chain of two LDS hand-offs; two workgroups per slice bring the former to 90 KB a chunk
 // (1900 tokens: 1.38 -> 0.97 us a chunk).
+// TWO: a grid of more than one workgroup per CU (several sequences, or many heads) is held to 128 VGPRs, so that
+// two fit on a CU: the next chunk's operands go to the registers of this one's as each is consumed.  The other form
+// has a second set for them, in 161 VGPRs, one workgroup per CU: 8 sequences of 25 tokens (1024 workgroups) 13.3 us
+// against 9.1 here, 3 of 40 (384) 7.7 against 5.5.
 constexpr int SCAN_T = 512;
-__global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict__ lu, const uint32_t* __restrict__ seqt,
+template <bool TWO>
+__global__ __launch_bounds__(SCAN_T, TWO ? 4 : 2) void k_gdn_scan(const uint32_t* __restrict__ lu, const uint32_t* __restrict__ seqt,
                                                      const uint32_t* __restrict__ chunkt, float* __restrict__ state,
                                                      int L, int load_default, size_t state_off, float* __restrict__ o,
                                                      const f16* __restrict__ big, f16* hist, size_t hist_off,
@@ -1107,7 +1112,8 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
     int c = cfirst;
     if (role == 0) {
         // ---- state role: V' = U - W S; S <- e^(G_last) S + KgT V'
-        WS set0, set1;
+        WS set0, second;
+        WS& set1 = TWO ? set0 : second;
         f16x8 kh[2][2], kl[2][2];
         float gl = 0.f;
         // the state: rows (2 wv + q2) 16 + 4 fg + r of column c0 + fr.  Its loads go through a buffer
@@ -1150,18 +1156,20 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
                 frag(o_kg + slot * (uint32_t)(KGF_H * 2), 2, wv * 2 + q2, s, kh[q2][s], kl[q2][s], vf);
         };
         auto chunk = [&](int cc, int p, const WS& cur, WS& nxt) {
-            load_u(nxt, cc + 1);
+            if constexpr (!TWO) load_u(nxt, cc + 1);
             lds_barrier();  // parity p holds this chunk's starting state; V' is free
             f32x4 av[3] = {z4, z4, z4};
             // k step s: its S fragments (all read at once), then the next chunk's W loads of step s, each
             // step a scheduling region of its own so that those loads are issued in four groups
             f16x8 sh8[4], sl8[4];
 #pragma unroll
-            for (int s = 0; s < 4; s++) s_frag(p, s, sh8[s], sl8[s]);
+            for (int s = 0; s < (TWO ? 1 : 4); s++) s_frag(p, s, sh8[s], sl8[s]);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                load_w_step(nxt, cc + 1, s);
+                if constexpr (!TWO) load_w_step(nxt, cc + 1, s);
+                else if (s < 3) s_frag(p, s + 1, sh8[s + 1], sl8[s + 1]);
                 mma3s(cur.wh[s], cur.wl[s], sh8[s], sl8[s], av);
+                if constexpr (TWO) load_w_step(nxt, cc + 1, s);
                 __builtin_amdgcn_sched_barrier(0);
             }
             // rows wv * 16 + fg * 4 .. + 3 of column fr: two 8-byte stores
@@ -1169,6 +1177,7 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
                 f32x4 v;
 #pragma unroll
                 for (int r = 0; r < 4; r++) v[r] = cur.ur[r] - (av[0][r] + av[1][r] + av[2][r]);
+                if constexpr (TWO) load_u(nxt, cc + 1);
                 f16x4 hi, lo;
                 split4(v, hi, lo);
                 *reinterpret_cast<f16x4*>(&Vh[fr * VP + wv * 16 + fg * 4]) = hi;
@@ -1181,18 +1190,20 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
             load_gl(cc + 1);  // e^(G_last) is consumed
             // S <- e^(G_last) S + KgT V': state row tiles 2w, 2w+1
             f32x4 as[2][3];
+            auto update = [&](int q2) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) S[q2][r] = g_c * S[q2][r] + (as[q2][0][r] + as[q2][1][r] + as[q2][2][r]);
+            };
 #pragma unroll
             for (int q2 = 0; q2 < 2; q2++) {
                 as[q2][0] = as[q2][1] = as[q2][2] = z4;
 #pragma unroll
                 for (int s = 0; s < 2; s++) mma3s(kh[q2][s], kl[q2][s], vh[s], vl[s], as[q2]);
                 load_kg(cc + 1, q2);  // Kg row tile q2 is consumed
+                if constexpr (TWO) update(q2);
                 __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int q2 = 0; q2 < 2; q2++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) S[q2][r] = g_c * S[q2][r] + (as[q2][0][r] + as[q2][1][r] + as[q2][2][r]);
+            if constexpr (!TWO) update(0), update(1);
             put_s(p ^ 1);
         };
 #pragma unroll
@@ -1215,7 +1226,8 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
         }
     } else {
         // ---- output role: o = Qg S + Qk V'
-        QS set0, set1;
+        QS set0, second;
+        QS& set1 = TWO ? set0 : second;
         f16x8 qkh[2], qkl[2];
         auto load_q_step = [&](QS& d, int cc, int s) {
             const uint32_t vf = cc < cend ? vfrag : OOB;
@@ -1239,11 +1251,13 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
             f32x4 ao[3] = {z4, z4, z4};
             f16x8 sh8[4], sl8[4];
 #pragma unroll
-            for (int s = 0; s < 4; s++) s_frag(p, s, sh8[s], sl8[s]);
+            for (int s = 0; s < (TWO ? 1 : 4); s++) s_frag(p, s, sh8[s], sl8[s]);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                load_q_step(nxt, cn, s);
+                if constexpr (!TWO) load_q_step(nxt, cn, s);
+                else if (s < 3) s_frag(p, s + 1, sh8[s + 1], sl8[s + 1]);
                 mma3s(cur.qh[s], cur.ql[s], sh8[s], sl8[s], ao);
+                if constexpr (TWO) load_q_step(nxt, cn, s);
                 __builtin_amdgcn_sched_barrier(0);
             }
             lds_barrier();  // V' complete
@@ -1261,7 +1275,7 @@ __global__ __launch_bounds__(SCAN_T) void k_gdn_scan(const uint32_t* __restrict_
                          __builtin_bit_cast(uint32_t, ao[0][r] + ao[1][r] + ao[2][r]));
             }
         };
-        const bool halves = !seqt && gridDim.z > 1;
+        const bool halves = !TWO && !seqt && gridDim.z > 1;  // never on a grid of more than 256
         const int first = cfirst + par, hop = halves ? 2 : 1;
 #pragma unroll
         for (int s = 0; s < 4; s++) load_q_step(set0, first, s);
@@ -1425,7 +1439,8 @@ void gdn_scan(const GdnShape& s, int L, const GdnWs& ws, float* state, const uin
     const bool in_place = !lu && load_default && !start;
     const int halves = !in_place && L > CH && s.H * (s.DV / DVS) * 2 <= 256 ? 2 : 1;
     if (!sg.seq) nseq = halves;
-    hipLaunchKernelGGL(k_gdn_scan, dim3(s.H, s.DV / DVS, nseq), dim3(SCAN_T), 0, st, lu, sg.seq, sg.chunk, state, L,
+    const auto f = s.H * (s.DV / DVS) * nseq > 256 ? k_gdn_scan<true> : k_gdn_scan<false>;
+    hipLaunchKernelGGL(f, dim3(s.H, s.DV / DVS, nseq), dim3(SCAN_T), 0, st, lu, sg.seq, sg.chunk, state, L,
                        load_default, state_off, o, big, hist, hist_off, start, s, ws);
     launched("gdn_scan");
 }

@@ -320,14 +320,20 @@ def test_gate_up_silu(sdamd, synth, oracle, M, exact, cfg):
     assert (err <= tol).all(), f"{(err > tol).sum()} beyond tolerance; max err {err.max()}"
 
 
+@pytest.mark.parametrize("L,load", [(1, True), (64, False), (129, True), (200, False), (256, True)])
+def test_gdn_of_more_workgroups_than_cus(sdamd, oracle, L, load):
+    """34 heads, 272 workgroups: the scan that keeps two of them on a CU, over 1 to 4 chunks, ragged and whole."""
+    test_gdn_halves_match_one_workgroup_per_slice(sdamd, oracle, L, load, H=34)
+
+
 @pytest.mark.parametrize("L,load", [(65, False), (128, True), (193, False), (320, False), (1025, True), (1088, True)])
-def test_gdn_halves_match_one_workgroup_per_slice(sdamd, oracle, L, load):
+def test_gdn_halves_match_one_workgroup_per_slice(sdamd, oracle, L, load, H=16):
     """Chunk counts 2 (ragged and whole), 4, 5 and 17 (ragged and whole) of a single sequence, whose scan runs as two
     workgroups per slice (output of every other chunk each), from nothing, from a state in place (one workgroup)
     and from a copy of it (from 1024 tokens on), against the oracle's sequential rule: 2e-4, as the other
     delta-rule tests."""
     rng = np.random.default_rng(L)
-    H, dk, dv = 16, 128, 128
+    dk, dv = 128, 128
     C = 2 * H * dk + H * dv
     qkv = rng.standard_normal((L, C)).astype(np.float32)
     big = rng.standard_normal((L, 2 * H)).astype(np.float16)
