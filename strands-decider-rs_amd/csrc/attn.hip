@@ -118,20 +118,6 @@ __global__ __launch_bounds__(256) void k_qk_prep(const f16* __restrict__ big, co
 constexpr float LOG2E = 1.4426950408889634f;
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Two f32 to packed f16 (round to nearest even), and p minus the low or high half of a packed pair in f32
-// (one v_fma_mix_f32 each, exact: the compiler converts each half on its own otherwise).
-__device__ __forceinline__ uint32_t cvt_pk(float a, float b) { return __builtin_bit_cast(uint32_t, f16x2{(f16)a, (f16)b}); }
-__device__ __forceinline__ float sub_lo(float p, uint32_t h) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(p));
-    return r;
-}
-__device__ __forceinline__ float sub_hi(float p, uint32_t h) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(p));
-    return r;
-}
-
 __device__ __forceinline__ float wave_max16(float v) {  // max over lanes {l, l^16, l^32, l^48}
     v = fmaxf(v, __shfl_xor(v, 16));
     return fmaxf(v, __shfl_xor(v, 32));
@@ -750,8 +736,8 @@ __global__ __launch_bounds__(256, 1) void k_attn_rows(const f16* __restrict__ Q,
     };
     auto psplit = [&](int u) {
         const float p0 = pe[2 * u], p1 = pe[2 * u + 1];
-        const uint32_t h2 = cvt_pk(p0, p1);
-        const f16x2 hi = __builtin_bit_cast(f16x2, h2), lo = __builtin_bit_cast(f16x2, cvt_pk(sub_lo(p0, h2), sub_hi(p1, h2)));
+        f16x2 hi, lo;
+        split2(p0, p1, hi, lo);
         l_run += p0;
         l_run += p1;
         ph[u >> 2][(2 * u) & 7] = hi[0];

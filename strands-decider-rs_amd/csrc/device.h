@@ -11,13 +11,46 @@ namespace {
 // (exact) for k = (0,1), (2,3), (4,5), (6,7): the nibble at bits 4p lands in the f16 mantissa as
 // 1024 + q for p = 0, 2 (and 4, 6 in the high half), as 1024 + 16 q for the others, so two masks per
 // 8-bit shift give all four pairs.
-// (a & m) | c in one v_and_or_b32 (the compiler otherwise emits separate and/or here).
+// Inline asm holds no vector instruction anywhere in these files: the compiler keeps the wait states
+// between an MFMA and a vector write of the registers it still reads as SrcC for its own instructions
+// only, not for those inside an asm.  Where it has to be led to one instruction, a constant or the
+// instruction's result goes through an empty asm that it cannot see through.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define OPAQUE_V(x) asm("" : "+v"(x))
+#define OPAQUE_S(x) asm("" : "+s"(x))
+#else
+#define OPAQUE_V(x) (void)(x)
+#define OPAQUE_S(x) (void)(x)
+#endif
+
+// (a & m) | c in one v_and_or_b32 (with constants that it sees, the compiler emits separate and/or here).
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t c) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(m), "s"(c));
-    return r;
+    OPAQUE_V(m);
+    OPAQUE_S(c);
+    return (a & m) | c;
 }
 
+// (v0, v1) = hi + lo as f16 pairs, hi rounded and lo the rounded rest: a packed convert for hi, the rest
+// v - hi (exact in f32) by one v_fma_mix_f32 on each half of hi's register, a packed convert for lo.  (A
+// subtraction, or a product with a -1 that the compiler sees, makes it convert each half on its own.)
+__device__ __forceinline__ void split2(float v0, float v1, f16x2& hi, f16x2& lo) {
+    uint32_t hb = __builtin_bit_cast(uint32_t, f16x2{(f16)v0, (f16)v1});
+    OPAQUE_V(hb);
+    hi = __builtin_bit_cast(f16x2, hb);
+    float m = -1.0f;
+    OPAQUE_S(m);
+    float r0 = __builtin_fmaf((float)hi[0], m, v0), r1 = __builtin_fmaf((float)hi[1], m, v1);
+    OPAQUE_V(r0);
+    OPAQUE_V(r1);
+    lo = f16x2{(f16)r0, (f16)r1};
+}
+
+// h s + b in f32 by one v_fma_mix_f32 on h's half of its register.
+__device__ __forceinline__ float mul_add_f16(f16 h, float s, float b) {
+    float r = __builtin_fmaf((float)h, s, b);
+    OPAQUE_V(r);
+    return r;
+}
 
 __device__ __forceinline__ void nib_pairs(uint32_t w, f16x2& p0, f16x2& p1, f16x2& p2, f16x2& p3) {
     const uint32_t w8 = w >> 8;

@@ -42,26 +42,14 @@ __device__ __forceinline__ float warp_sum8(float v) {  // sum over aligned group
     return v;
 }
 
-// v = hi + lo with hi = f16(v) and lo = f16(v - hi), in pairs: one packed convert for two hi, the
-// residual v - f32(hi) (exact in f32) by one v_fma_mix_f32 each (hi's half as an f16 operand, times
-// -1, plus v), one packed convert for two lo: 12 VALU per 8 values instead of 32.
+// v = hi + lo with hi = f16(v) and lo = f16(v - hi), in pairs: 12 VALU per 8 values instead of 32.
 __device__ __forceinline__ void split8(const float* v, f16x8& hi, f16x8& lo) {
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-        const f16x2 h = f16x2{(f16)v[e], (f16)v[e + 1]};
-        float r0, r1;
-#if defined(__HIP_DEVICE_COMPILE__)
-        const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hb), "v"(v[e]));
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hb), "v"(v[e + 1]));
-#else
-        r0 = v[e] - (float)h[0];
-        r1 = v[e + 1] - (float)h[1];
-#endif
-        hi[e] = h[0];
-        hi[e + 1] = h[1];
-        lo[e] = (f16)r0;
-        lo[e + 1] = (f16)r1;
+        f16x2 h, l;
+        split2(v[e], v[e + 1], h, l);
+        hi[e] = h[0], hi[e + 1] = h[1];
+        lo[e] = l[0], lo[e + 1] = l[1];
     }
 }
 
@@ -69,21 +57,10 @@ __device__ __forceinline__ void split8(const float* v, f16x8& hi, f16x8& lo) {
 __device__ __forceinline__ void split4(const f32x4& v, f16x4& hi, f16x4& lo) {
 #pragma unroll
     for (int e = 0; e < 4; e += 2) {
-        const f16x2 h = f16x2{(f16)v[e], (f16)v[e + 1]};
-        float r0, r1;
-#if defined(__HIP_DEVICE_COMPILE__)
-        const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-        const float v0 = v[e], v1 = v[e + 1];
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hb), "v"(v0));
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hb), "v"(v1));
-#else
-        r0 = v[e] - (float)h[0];
-        r1 = v[e + 1] - (float)h[1];
-#endif
-        hi[e] = h[0];
-        hi[e + 1] = h[1];
-        lo[e] = (f16)r0;
-        lo[e + 1] = (f16)r1;
+        f16x2 h, l;
+        split2(v[e], v[e + 1], h, l);
+        hi[e] = h[0], hi[e + 1] = h[1];
+        lo[e] = l[0], lo[e + 1] = l[1];
     }
 }
 

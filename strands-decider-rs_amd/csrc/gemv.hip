@@ -312,21 +312,12 @@ __device__ __forceinline__ void code_pairs(const typename BlkT<BITS>::T& w, int 
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             p[k] = and_or(x >> (4 * k), 0x00030003u, EXP);
-            if constexpr (BITS == 3) p[k] |= (h >> (2 * k)) & 0x00040004u;
+            if constexpr (BITS == 3) {
+                OPAQUE_V(p[k]);  // (not merged into two ands and a three-way or)
+                p[k] |= (h >> (2 * k)) & 0x00040004u;
+            }
         }
     }
-}
-
-// a's low or high f16 half times b plus c, in f32 (one rounding)
-__device__ __forceinline__ float mix_lo(uint32_t a, float b, float c) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float mix_hi(uint32_t a, float b, float c) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
 }
 
 template <int BITS, bool ASYM, int MT, bool PARTIAL, int KH>
@@ -399,12 +390,8 @@ __global__ __launch_bounds__(256 * KH) void k_gemm_fmt(const f16* __restrict__ A
             if constexpr (ASYM) {
                 const float s32 = (float)sc, b32 = (float)__builtin_bit_cast(f16, (uint16_t)bb[slot]);
                 const f16x2 c = __builtin_bit_cast(f16x2, p[k]) - f16x2{(f16)1024.f, (f16)1024.f};
-                const uint32_t cb = __builtin_bit_cast(uint32_t, c);
-                const float v0 = mix_lo(cb, s32, b32), v1 = mix_hi(cb, s32, b32);
-                h = f16x2{(f16)v0, (f16)v1};
-                const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-                const float r0 = mix_lo(hb, -1.0f, v0), r1 = mix_hi(hb, -1.0f, v1);
-                l = f16x2{(f16)r0, (f16)r1};
+                const float v0 = mul_add_f16(c[0], s32, b32), v1 = mul_add_f16(c[1], s32, b32);
+                split2(v0, v1, h, l);
             } else {
                 constexpr float Z = 1024.f + (float)(1 << (BITS - 1));
                 const f16x2 c = __builtin_bit_cast(f16x2, p[k]) - f16x2{(f16)Z, (f16)Z}, sc2 = f16x2{sc, sc};
