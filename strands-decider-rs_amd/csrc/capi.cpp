@@ -399,12 +399,12 @@ int sd_op_gdn(const void* qkv, const void* big, int stride, int a_off, int b_off
         const sd::GdnShape s{H, dk, dv, stride, a_off, b_off, 0, 2 * H * dk + H * dv};
         OpWs& w = op_ws();
         std::lock_guard<std::mutex> lock(w.mu);
-        // A long continuation starts from a copy of the state, which the scan then writes from two
-        // workgroups per slice (1024 tokens 38.5 -> 37.6 us,
-        // 1900 66.7 -> 62.7, the copy included; 769 tokens would lose 0.8).
+        // A long continuation starts from a copy of the state, where the scan then runs as two workgroups per
+        // slice (16 heads, the copy included: 1024 tokens 38.5 -> 37.6 us, 1900 66.7 -> 62.7; 769 tokens would
+        // lose 0.8; 32 heads, whose scan stays at one: 1024 tokens 55.1 without the copy, 57.5 with it).
         const size_t ws_bytes = (sd::gdn_ws_bytes(L, s) + 255) & ~size_t(255), state_bytes = (size_t)H * dk * dv * 4;
-        const bool copy = load_state && L >= 1024 && reinterpret_cast<uintptr_t>(state) % 16 == 0;
-        const size_t need = ws_bytes + state_bytes;
+        const bool copy = load_state && L >= 1024 && sd::gdn_scan_halves(s, L) && reinterpret_cast<uintptr_t>(state) % 16 == 0;
+        const size_t need = ws_bytes + (copy ? state_bytes : 0);
         if (need > w.gdn_bytes) {
             if (w.gdn) SD_HIP(hipFree(w.gdn));
             w.gdn = nullptr;

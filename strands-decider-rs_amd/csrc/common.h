@@ -203,7 +203,9 @@ void gdn_prep(const float* qkvc, const f16* big, const GdnShape& s, const float*
 // names one); with lu null, load_default decides.  Every sequence starts from that state; the final
 // state is written to `state` only for a single sequence (sg.seq null).  nseq = sequence grid size.
 // hist (nullable) is updated from big at the end (the reference's hist_update; single sequence
-// only), its old rows from the prefix's history.
+// only), its old rows from the prefix's history.  start (nullable) = the state it starts from where lu is null
+// and load_default set, else `state` itself.
+bool gdn_scan_halves(const GdnShape& s, int L);  // a single sequence's two-workgroup form fits (if not in place)
 void gdn_scan(const GdnShape& s, int L, const GdnWs& ws, float* state, const uint32_t* lu, int load_default, float* o,
               const Segs& sg, int nseq, hipStream_t st, size_t state_off = 0, f16* hist = nullptr,
               const f16* big = nullptr, size_t hist_off = 0, const float* start = nullptr);

@@ -1403,18 +1403,21 @@ void gdn_prep(const float* qkvc, const f16* big, const GdnShape& s, const float*
     launched("gdn_prep");
 }
 
+// One sequence of several chunks on a grid that leaves half the CUs idle runs as two workgroups per slice
+// (prep + scan on MI355X at 16 heads, one against two: 512 tokens 30.2 -> 29.1 us, 1024 38.5 -> 34.9, 1900
+// 66.7 -> 60.0, 3000 103 -> 93).
+bool gdn_scan_halves(const GdnShape& s, int L) { return L > CH && s.H * (s.DV / DVS) * 2 <= 256; }
+
 void gdn_scan(const GdnShape& s, int L, const GdnWs& ws, float* state, const uint32_t* lu, int load_default, float* o,
               const Segs& sg, int nseq, hipStream_t st, size_t state_off, f16* hist, const f16* big, size_t hist_off,
               const float* start) {
     SD_CHECK(s.DK == 128 && s.DV == 128, "gated delta net: only 128-wide key/value heads are supported");
     SD_CHECK(!sg.seq || (lu && sg.chunk), "gdn_scan: several sequences need lu and the chunk table");
     SD_CHECK(!hist || (!sg.seq && big), "gdn_scan: the history update needs one sequence and big");
-    // One sequence of several chunks on a grid that leaves half the CUs idle runs as two workgroups per slice
-    // (prep + scan on MI355X, one against two: 512 tokens 30.2 -> 29.1 us, 1024 38.5 -> 34.9, 1900 66.7 -> 60.0,
-    // 3000 103 -> 93).  Not where the state it starts from is the one it writes: the first may have written
-    // it before the second starts.  (With lu a single sequence starts from a snapshot or from nothing.)
+    // Two workgroups per slice, but not where the state it starts from is the one it writes: the first may have
+    // written it before the second starts.  (With lu a single sequence starts from a snapshot or from nothing.)
     const bool in_place = !lu && load_default && !start;
-    const int halves = !in_place && L > CH && s.H * (s.DV / DVS) * 2 <= 256 ? 2 : 1;
+    const int halves = !in_place && gdn_scan_halves(s, L) ? 2 : 1;
     if (!sg.seq) nseq = halves;
     const auto f = s.H * (s.DV / DVS) * nseq > 256 ? k_gdn_scan<true> : k_gdn_scan<false>;
     hipLaunchKernelGGL(f, dim3(s.H, s.DV / DVS, nseq), dim3(SCAN_T), 0, st, lu, sg.seq, sg.chunk, state, L,

@@ -320,9 +320,10 @@ def test_gate_up_silu(sdamd, synth, oracle, M, exact, cfg):
     assert (err <= tol).all(), f"{(err > tol).sum()} beyond tolerance; max err {err.max()}"
 
 
-@pytest.mark.parametrize("L,load", [(1, True), (64, False), (129, True), (200, False), (256, True)])
+@pytest.mark.parametrize("L,load", [(1, True), (64, False), (129, True), (200, False), (256, True), (1100, True)])
 def test_gdn_of_more_workgroups_than_cus(sdamd, oracle, L, load):
-    """34 heads, 272 workgroups: the scan that keeps two of them on a CU, over 1 to 4 chunks, ragged and whole."""
+    """34 heads, 272 workgroups: the scan that keeps two of them on a CU, over 1 to 18 chunks, ragged and whole (a
+    loaded state is read in place at every length)."""
     test_gdn_halves_match_one_workgroup_per_slice(sdamd, oracle, L, load, H=34)
 
 
