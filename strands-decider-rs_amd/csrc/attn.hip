@@ -1000,23 +1000,30 @@ size_t attn_ws_floats(int rows, const AttnShape& s) { return (size_t)ATTN_KS_MAX
 //   k_attn          17.0       18.7        27.8        32.3         19.1      20.2      47.9       119
 //   k_attn_rows     18.4       19.3-20.6   22.3        29.4         16.1      19.0      26.7       51.1
 // A tile of 32 (query, head) rows has half as many workgroups as k_attn's 16 queries of a head, so up to 128
-// rows (64 of k_attn's tiles) the latter's shorter chains win.
-//  * k_attn splits the keys while its grid stays within one workgroup per CU (70 rows: 18.2 us in 4 splits,
-//    21.0 in 8).
+// rows the latter's shorter chains win.  From 129 to 256 rows they also do (us, k_attn | k_attn_rows):
+//  * with few heads over a prefix, where 8 splits of k_attn are at most one workgroup per CU (32 tiles): 2
+//    query and 2 kv heads, 160 + 512: 16.2 in 8 splits | 17.3 in 4, 16.9 in 8; + 2048 19.8 | 20.7; 250 + 512:
+//    17.8 | 18.2.  From 36 tiles on k_attn has 4: 4 and 1 heads, 129 + 2048 22.6 | 21.2, + 3800 29.0 | 25.9;
+//  * without a prefix, the keys being the rows, unsplit and within one workgroup per CU: 8 and 2 heads, 129
+//    rows 14.1 | 15.4, 250 15.3 | 16.1; 16 and 1 heads, 250 rows 15.8 | 16.6 (32 and 8, 288 tiles: 21.0 | 17.3).
+// Where k_attn runs up to 128 rows, or over a prefix:
+//  * it splits the keys while its grid stays within one workgroup per CU (70 rows: 18.2 us in 4 splits, 21.0
+//    in 8).
 //  * k_attn_rows up to 256 rows splits them only over a prefix, in 4 up to 48 tiles (200 + 2048: 25.2 us in 4
 //    splits, 28.3 in 2, 33.0 in 1; 128 + 512: 19.3 / 19.5 / 18.3) and in 2 up to 64 (250 + 512: 24.1 / 23.2 /
 //    20.5, + 2048: 26.7 / 29.4 / 33.4).
 AttnPlan attn_plan(int L, const AttnShape& s, bool prefix) {
     const int G = s.HQ / s.HK;
     AttnPlan p;
-    p.rows = L > 128 && G <= 32 && (G & (G - 1)) == 0;
-    if (L > ATTN_SPLIT_ROWS) return p;
+    const int tiles16 = (L + BQ - 1) / BQ * s.HQ;  // of k_attn
+    const bool few = L <= ATTN_SPLIT_ROWS && tiles16 * (prefix ? ATTN_KS_MAX : 1) <= 256;
+    p.rows = L > 128 && !few && G <= 32 && (G & (G - 1)) == 0;
+    if (L > ATTN_SPLIT_ROWS || (L > 128 && !prefix)) return p;
     if (p.rows) {
         const int tiles = (L * G + 31) / 32 * s.HK;
-        p.ks = !prefix || tiles > 64 ? 1 : tiles > 48 ? 2 : 4;
+        p.ks = tiles > 64 ? 1 : tiles > 48 ? 2 : 4;
     } else {
-        const int tiles = (L + BQ - 1) / BQ * s.HQ;
-        while (p.ks < ATTN_KS_MAX && tiles * p.ks * 2 <= 256) p.ks *= 2;
+        while (p.ks < ATTN_KS_MAX && tiles16 * p.ks * 2 <= 256) p.ks *= 2;
     }
     return p;
 }

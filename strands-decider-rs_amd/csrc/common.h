@@ -250,6 +250,7 @@ constexpr int ATTN_SPLIT_ROWS = 256;
 struct AttnPlan {
     bool rows = false;
     int ks = 1;
+    bool operator!=(const AttnPlan& o) const { return rows != o.rows || ks != o.ks; }
 };
 AttnPlan attn_plan(int L, const AttnShape& s, bool prefix);
 size_t attn_ws_floats(int rows, const AttnShape& s);

@@ -649,9 +649,9 @@ Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, 
                             : 0;
     // the attention's plan: the prefix bit is part of the key only where it changes it
     const AttnShape head{cfg.hq, cfg.hk, cfg.hd, cfg.rd, 0, SD_CONTEXT};
-    const bool split_bit = !attn_layers.empty() && prefix && attn_plan(L, head, true).ks != attn_plan(L, head, false).ks;
-    const uint64_t key = (uint64_t)(cache_only ? 1u : 0u) << 63 | (uint64_t)(split_bit ? 1u : 0u) << 62 | (uint64_t)compact << 46 | (uint64_t)tree << 32 |
-                         (uint64_t)L << 8 | (uint64_t)nseq << 1 | (short_seqs ? 1u : 0u);
+    const bool prefix_bit = !attn_layers.empty() && prefix && attn_plan(L, head, true) != attn_plan(L, head, false);
+    const uint64_t key = (uint64_t)(cache_only ? 1u : 0u) << 63 | (uint64_t)(prefix_bit ? 1u : 0u) << 62 |
+                         (uint64_t)compact << 46 | (uint64_t)tree << 32 | (uint64_t)L << 8 | (uint64_t)nseq << 1 | (short_seqs ? 1u : 0u);
     auto it = plans.find(key);
     if (it != plans.end()) {
         it->second.used = ++plan_clock;
@@ -796,7 +796,7 @@ Plan& Engine::plan(int L, int nseq, bool short_seqs, int tree, bool cache_only, 
                 qk_prep(P.big, as, W.q_norm, W.k_norm, rp, L, luv, sg, qbuf, W.kc, W.vc, s);
             }});
             if (cache_end) break;
-            const AttnPlan ap = attn_plan(L, as, split_bit);
+            const AttnPlan ap = attn_plan(L, as, prefix_bit);
             SD_CHECK(ap.ks == 1 || L <= P.attn_rows, "attention: the key-split workspace is too small");
             steps.push_back({"attn", [=](hipStream_t s) {
                 attention_split(qbuf, W.kc, W.vc, P.big, as, L, luv, sg, ap, P.attn_ws, P.o, s, W.q_norm, rp);

@@ -239,8 +239,8 @@ struct Engine {
     // tree > 0: sequence 0 is a state of `tree` rows and sequences 1 .. nseq - 1 continue from it
     // (their own rows attend to its rows, their delta rule starts from its final state), each as its
     // own forward from the state's snapshot would; see ask_tree.
-    // prefix: the forward continues from a snapshot (it only picks the attention's key splits; a plan runs
-    // with any prefix or none).
+    // prefix: the forward continues from a snapshot (it only picks the attention's kernel and key splits; a
+    // plan runs with any prefix or none).
     Plan& plan(int L, int nseq = 0, bool short_seqs = false, int tree = 0, bool cache_only = false, int rows_read = 0,
                bool prefix = false);
     void upload(const uint32_t* ids, size_t n, const size_t* rows, size_t n_rows, size_t P, bool has_cache,

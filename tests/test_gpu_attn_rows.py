@@ -59,16 +59,18 @@ def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0):
                            f"max {np.abs(got - want).max():.3g}")
 
 
-@pytest.mark.parametrize("L,P", [(129, 0), (136, 31), (150, 0), (159, 64), (193, 33), (257, 95), (300, 0), (513, 700)])
+@pytest.mark.parametrize("L,P", [(129, 0), (136, 31), (150, 0), (159, 64), (193, 33), (256, 0), (257, 95), (264, 0), (300, 0), (513, 700)])
 def test_rows_kernel_edges(sdamd, oracle, L, P):
     """Ragged last tiles (8 queries each), prefixes that end inside a 32-key block, splits of 1, 2 and 4."""
     check(sdamd, oracle, L + P, 8, 2, L, P)
 
 
 @pytest.mark.parametrize("hq,hk", [(2, 2), (4, 2), (8, 1), (16, 1), (6, 2)])
-def test_rows_kernel_groups(sdamd, oracle, hq, hk):
-    """1, 2, 8 and 16 query heads per kv head (32, 16, 4 and 2 queries per tile); 3 take the other kernel."""
-    check(sdamd, oracle, 7 * hq + hk, hq, hk, 141, 50)
+@pytest.mark.parametrize("L,P", [(141, 50), (269, 50)])
+def test_rows_kernel_groups(sdamd, oracle, hq, hk, L, P):
+    """1, 2, 8 and 16 query heads per kv head (32, 16, 4 and 2 queries per tile); 3 take the other kernel, as 2
+    query heads do up to 256 rows."""
+    check(sdamd, oracle, 7 * hq + hk, hq, hk, L, P)
 
 
 @pytest.mark.parametrize("L,P", [(160, 0), (160, 70), (300, 33)])

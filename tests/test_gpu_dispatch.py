@@ -5,6 +5,30 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
+ROWS, QUERIES = "32 (query, head) rows per workgroup", "16 queries of a head per workgroup"
+
+
+@pytest.mark.parametrize("hq,hk,L,P,kernel,ks", [
+    (8, 2, 128, 512, QUERIES, 4), (8, 2, 129, 512, ROWS, 4), (8, 2, 200, 512, ROWS, 2), (8, 2, 256, 2048, ROWS, 2),
+    (8, 2, 257, 512, ROWS, 1), (16, 2, 250, 512, ROWS, 1),
+    (2, 2, 129, 512, QUERIES, 8), (2, 2, 256, 2048, QUERIES, 8), (2, 2, 257, 512, ROWS, 1), (4, 1, 129, 512, ROWS, 4),
+    (8, 2, 128, 0, QUERIES, 4), (8, 2, 129, 0, QUERIES, 1), (8, 2, 256, 0, QUERIES, 1), (8, 2, 257, 0, ROWS, 1),
+    (16, 1, 256, 0, QUERIES, 1), (32, 8, 129, 0, ROWS, 1), (2, 2, 256, 0, QUERIES, 1), (6, 2, 129, 0, QUERIES, 1),
+    (6, 2, 200, 512, QUERIES, 2), (6, 2, 300, 512, QUERIES, 1)])
+def test_attention_kernel_and_splits(sdamd, hq, hk, L, P, kernel, ks):
+    """Which attention kernel runs, in how many key splits (a combine follows more than one)."""
+    from launches import launches
+    hd, ctx, stride = 256, 4096, 2 * hq * 256 + 2 * hk * 256
+    big, out, q = (torch.zeros(n, device="cuda").half() for n in (L * stride, L * hq * hd, L * hq * hd))
+    w, rope = torch.ones(hd, device="cuda"), torch.zeros(ctx, 32, 2, device="cuda")
+    k, v = (torch.zeros(hk * ctx * hd, device="cuda").half() for _ in range(2))
+    got = launches(sdamd, lambda s: sdamd.op_attention(big.data_ptr(), stride, w.data_ptr(), w.data_ptr(), rope.data_ptr(), L, P, hq,
+                                                       hk, hd, 64, q.data_ptr(), k.data_ptr(), v.data_ptr(), ctx, out.data_ptr(), s))
+    assert len(got) == (4 if ks > 1 else 3), got  # two integers, the rows' k and v, attention, the combine
+    grid = (hk, -(-L * (hq // hk) // 32), ks) if kernel is ROWS else (-(-L // 16), hq, ks)
+    assert got[2][0] == grid, got
+
+
 @pytest.mark.parametrize("H,L,load,copied,halves", [(16, 1024, True, True, 2), (16, 1023, True, False, 1), (16, 1024, False, False, 2),
                                                     (17, 1024, True, False, 1), (34, 1100, True, False, 1)])
 def test_gdn_copies_its_state_only_for_two_workgroups_per_slice(sdamd, H, L, load, copied, halves):
