@@ -1111,14 +1111,22 @@ GemmPlan gemm_w4_plan(int M, int N, int K, bool exact, bool partial_ok, size_t m
         const bool one_round = (size_t)((N + 127) / 128) * ((M + 95) / 96) <= 256;
         // Above 2560 rows two column tiles per wave: (4,2) reads an A fragment from LDS for two MFMAs, where
         // (4,1), (3,1) and (2,1) read one for each and need the LDS's whole 128 bytes a clock at the MFMAs'
-        // full rate (counters at 4096 x 12288: MFMAs busy 66% of the clocks for (4,2), 52% for (4,1)).  It pays
-        // once its 128 x 256 tiles are about 1.6 per CU.  us at M = 3000: gate_up 148 against 159 for (4,1),
-        // in_proj 113 / 123 for (3,1), qkv 62 / 72 for (4,1); with fewer tiles and k halves (one workgroup of
-        // 8 waves per CU) down 82.5 / 88 and out_proj 33.3 / 34.7 for (4,1); qkv at 1777 rows, 280 tiles: 51
-        // against 41 for (3,1).
+        // full rate.  It pays once its 128 x 256 tiles are about 1.6 per CU.  us at M = 3000: gate_up 150
+        // against 161 for (4,1), in_proj 112 / 124 for (3,1), qkv 63 / 72 for (4,1); qkv at 1777 rows, 280 tiles:
+        // 51 against 41 for (3,1).  Not
+        //  * below K = 1024, whose few steps do not pay for the larger tiles' prologue and output: 9216 x 512 at
+        //    2700 rows 37.5 against 34.3 for (3,1), 16384 x 256 40.0 / 38.4 for (4,1); 4096 x 1024 at 3200 rows
+        //    33.4 / 38.1;
+        //  * where (3,1) is the alternative and they are a little more than two per CU: 7168 x 2048, 588 tiles
+        //    88.3 / 81.9, 616 tiles 87.8 / 91.0.
+        // With fewer tiles and k halves, one workgroup of 8 waves per CU: down 83.1 against 90.9 for (4,1), out_proj
+        // 34.6 / 36.8 (2561 rows: 31.9 to 32.7 / 31.1 to 32.4 from box to box).  Not
+        //  * with more than three CUs in eight idle: 1024 x 1024, 128 tiles 19.0 / 14.1, 1024 x 6144 80.7 / 61.9, 1536
+        //    x 2048, 132 tiles 31.7 / 30.5; 1280 x 4096, 160 tiles 55.3 / 59.8;
+        //  * below K = 2048: 2048 x 1024 at 2561 rows 20.8 / 19.0, 3072 x 1024 24.6 / 22.0, 2048 x 1536 26.9 / 26.0.
         const size_t tiles42 = (size_t)((N + 255) / 256) * ((M + 127) / 128);
-        if (M > 2560 && tiles42 >= 400) p.cfg = W42;
-        else if (M > 2560 && halves_ok && tiles42 >= 128 && tiles42 <= 256) p.cfg = W42h;
+        if (M > 2560 && K >= 1024 && tiles42 >= (N >= 7000 ? 600 : 400)) p.cfg = W42;
+        else if (M > 2560 && K >= 2048 && halves_ok && tiles42 >= 160 && tiles42 <= 256) p.cfg = W42h;
         else if (N >= 10000) p.cfg = M >= 1792 ? W41 : W31;
         else if (N >= 7000) p.cfg = W31;
         else if (N >= 4000) p.cfg = W41;

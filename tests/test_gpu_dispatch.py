@@ -29,6 +29,19 @@ def test_attention_kernel_and_splits(sdamd, hq, hk, L, P, kernel, ks):
     assert got[2][0] == grid, got
 
 
+@pytest.mark.parametrize("M,N,K,rows,columns,threads", [
+    (2561, 5120, 2048, 128, 256, 256), (2561, 7168, 2048, 96, 128, 256), (2800, 7168, 2048, 128, 256, 256),  # two column tiles per wave
+    (2700, 9216, 512, 96, 128, 256), (2700, 16384, 256, 128, 128, 256), (3200, 4096, 1024, 128, 256, 256),
+    (2561, 2048, 2048, 128, 256, 512), (2560, 2048, 2560, 128, 128, 256), (4096, 1280, 4096, 128, 256, 512),  # and k halves
+    (4096, 1024, 1024, 128, 128, 256), (2816, 1536, 2048, 128, 128, 256), (2561, 2048, 1024, 128, 128, 256)])
+def test_long_prefill_tiles(sdamd, M, N, K, rows, columns, threads):
+    """The tile of an int4 matmul above 2560 rows: its grid and workgroup size."""
+    from launches import launches
+    a, w, s, y = (torch.zeros(n, device="cuda").half() for n in (M * K, N * K // 4, N * K // 32, M * N))
+    got = launches(sdamd, lambda st: sdamd.op_matmul(a.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), M, N, K, False, -1, True, st))
+    assert got == [((-(-N // columns), -(-M // rows), 1), threads)], got
+
+
 @pytest.mark.parametrize("H,L,load,copied,halves", [(16, 1024, True, True, 2), (16, 1023, True, False, 1), (16, 1024, False, False, 2),
                                                     (17, 1024, True, False, 1), (34, 1100, True, False, 1)])
 def test_gdn_copies_its_state_only_for_two_workgroups_per_slice(sdamd, H, L, load, copied, halves):
