@@ -526,8 +526,10 @@ GemvPlan gemv_plan(int M, int N, int K, bool tiled, int out, size_t max_part_ele
     // Six formats of int2 to int4, K = 2048, k_gemv's time over this kernel's (least, most):
     //   N = 5120: 8 rows 0.76, 0.99  16 rows 0.87, 1.11  17 rows 1.02, 1.36  33 rows 1.32, 1.71
     //   N = 8256: 4 rows 0.96, 1.29   8 rows 1.04, 1.34  17 rows 1.44, 1.85;  N = 12288: 4 rows 0.99, 1.32  8 rows 1.06, 1.35
+    // A single step (K = 128), half of whose two parts idle, from two workgroups per CU: 4096 columns, int4
+    // asymmetric, 64 rows 6.77 | 6.94, 65 rows (768) 9.86 | 7.01.
     const size_t blocks = (size_t)((N + 15) / 16) * rb;
-    if (!tiled && out != 2 && K % 128 == 0 && blocks > 256 && (M > 16 || (M >= 8 && blocks > 512))) {
+    if (!tiled && out != 2 && K % 128 == 0 && blocks > 256 && (blocks > 512 ? M >= 8 : M > 16 && K > 128)) {
         const size_t cols = (N + 63) / 64, g2 = cols * ((M + 31) / 32), g4 = cols * ((M + 63) / 64);
         p.rows = g2 <= 256 ? 2 : 4;
         p.kh = p.rows == 2 || g4 <= 256 ? 2 : 1;

@@ -42,6 +42,18 @@ def test_long_prefill_tiles(sdamd, M, N, K, rows, columns, threads):
     assert got == [((-(-N // columns), -(-M // rows), 1), threads)], got
 
 
+@pytest.mark.parametrize("M,N,K,many", [(7, 8256, 256, False), (8, 8192, 256, False), (8, 8256, 256, True), (16, 5120, 256, False),
+                                        (17, 4096, 256, False), (17, 4112, 256, True), (64, 4096, 256, True),
+                                        (64, 4096, 128, False), (65, 4096, 128, True), (300, 2048, 192, False)])
+def test_other_formats_at_many_rows(sdamd, M, N, K, many):
+    """The kernel that dequantizes a weight once per 32 or 64 rows (64 columns per workgroup; 16 for the other)."""
+    from launches import launches
+    a, w, s, y = (torch.zeros(n, device="cuda").half() for n in (M * K, N * K * 3 // 16, N * K // 32, M * N))
+    got = launches(sdamd, lambda st: sdamd.op_matmul_fmt(a.data_ptr(), w.data_ptr(), s.data_ptr(), None, y.data_ptr(), M, N, K, 3, 32,
+                                                         False, st))
+    assert len(got) == 1 and got[0][0][0] == -(-N // (64 if many else 16)), got
+
+
 @pytest.mark.parametrize("H,L,load,copied,halves", [(16, 1024, True, True, 2), (16, 1023, True, False, 1), (16, 1024, False, False, 2),
                                                     (17, 1024, True, False, 1), (34, 1100, True, False, 1)])
 def test_gdn_copies_its_state_only_for_two_workgroups_per_slice(sdamd, H, L, load, copied, halves):
