@@ -18,9 +18,11 @@ def dev(a):
     return torch.from_numpy(a.view(np.uint8).reshape(-1).copy()).cuda()
 
 
-def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0):
+def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0, own=False):
     """P prefix rows straight in the cache, then L rows; out within 2 f16 ulp + 1e-3 of the oracle (scores,
-    softmax and P V in f32 against the oracle's f64 softmax: the bound of the other attention tests)."""
+    softmax and P V in f32 against the oracle's f64 softmax: the bound of the other attention tests).  own: the
+    oracle's attention takes the queries and the cache that the GPU prepared, so that only scores, softmax and P V
+    differ."""
     from conftest import f16_ulp
     rng = np.random.default_rng(seed)
     qw = (gain * (1 + 0.1 * rng.standard_normal(HD))).astype(np.float32)
@@ -39,13 +41,17 @@ def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0):
         assert dK.data_ptr() % 16 == shift and dV.data_ptr() % 16 == shift
     dbig, dqw, dkw, drope = dev(big), dev(qw), dev(kw), dev(rope)
     dQ = torch.zeros(hq * L * HD * 2, dtype=torch.uint8, device="cuda")
-    dout = torch.zeros(L * hq * HD * 2, dtype=torch.uint8, device="cuda")
+    dout = torch.full((L * hq * HD * 2,), 0xFF, dtype=torch.uint8, device="cuda")  # NaN until written
     sdamd.op_attention(dbig.data_ptr(), stride, dqw.data_ptr(), dkw.data_ptr(), drope.data_ptr(), L, P, hq, hk, HD, rd,
                        dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), CTX, dout.data_ptr())
     torch.cuda.synchronize()
     Q = np.empty((hq, L, HD), np.uint16)
     o.lib().or_qk_prep(o.P(big.view(np.uint16)), I(stride), o.P(qw), o.P(kw), o.P(rope), I(L), I(P), I(CTX), I(hq),
                        I(hk), I(HD), I(rd), o.P(Q), o.P(oK), o.P(oV))
+    if own:
+        Q = dQ.cpu().numpy().view(np.uint16).reshape(hq, L, HD).copy()
+        oK = dK.cpu().numpy().view(np.uint16).reshape(hk, CTX // 32, HD // 32, 32, 32).transpose(0, 1, 3, 2, 4).reshape(hk, CTX, HD).copy()
+        oV = dV.cpu().numpy().view(np.uint16).reshape(hk, CTX // 32, HD, 32).transpose(0, 1, 3, 2).reshape(hk, CTX, HD).copy()
     out = np.empty((L, hq * HD), np.uint16)
     o.lib().or_attn(o.P(Q), o.P(oK), o.P(oV), o.P(big.view(np.uint16)), I(stride), I(L), I(P), I(CTX), I(hq), I(hk),
                     I(HD), o.P(out))
@@ -54,7 +60,14 @@ def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0):
     # a large gain on q: the 1-ulp f16 difference of a query (2^-11) moves its scores (up to ~100) by ~0.05,
     # which is a factor e^0.05 between two keys' weights
     extra = 1e-3 if gain == 1.0 else 5e-2
-    bad = np.abs(got - want) > 2.0 * f16_ulp(want) + extra
+    if own:
+        # a score is 256 f32 products and sums, off by about 16 x 2^-24 of the sum of their magnitudes, which moves a
+        # weight and the weights' sum by as much relative to itself, and the output by twice that of the values
+        q, k, v = (np.abs(o.h2f(x)[:, :P + L]) for x in (Q, oK, oV))
+        sums = max(float((q[h] @ k[h // (hq // hk)].T).max()) / 16 for h in range(hq))
+        extra = 2 * 16 * 2.0 ** -24 * sums * float(v.max())
+        assert extra < 1e-2
+    bad = ~(np.abs(got - want) <= 2.0 * f16_ulp(want) + extra)
     assert not bad.any(), (f"L={L} P={P} heads {hq}/{hk}: {int(bad.sum())} outputs off, "
                            f"max {np.abs(got - want).max():.3g}")
 
@@ -86,8 +99,11 @@ def test_rows_kernel_reads_prepared_queries(sdamd, oracle):
 
 def test_rows_kernel_raises_its_maximum(sdamd, oracle):
     """Queries scaled by 12: scores of a standard deviation of 12 in the exponent, so the running maximum
-    rises by more than the kernel's slack again and again."""
+    rises by more than the kernel's slack again and again.  From the GPU's own queries (the kernel that reads
+    them prepared) the oracle's scores are the same but for the f32 sums."""
     check(sdamd, oracle, 9, 8, 2, 400, 100, gain=12.0)
+    check(sdamd, oracle, 9, 8, 2, 400, 100, gain=12.0, rd=32, own=True)
+    check(sdamd, oracle, 10, 8, 2, 200, 900, gain=12.0, rd=32, own=True)
 
 
 def test_a_tile_of_one_query_is_as_fast_as_one_of_two(sdamd):

@@ -31,6 +31,11 @@ def empty(nbytes):
     return torch.zeros(max(nbytes, 16), dtype=torch.uint8, device="cuda")
 
 
+def unset(nbytes):
+    """An output that reads as NaN until it is written."""
+    return torch.full((nbytes,), 0xFF, dtype=torch.uint8, device="cuda")
+
+
 def host(t, dtype, shape):
     torch.cuda.synchronize()
     return t.cpu().numpy().view(dtype)[:int(np.prod(shape))].reshape(shape)
@@ -41,7 +46,7 @@ def within(got, want, ulps=1.0, extra=0.0, what=""):
     want = np.asarray(want, np.float32)
     err = np.abs(got - want)
     tol = ulps * f16_ulp(want) * 1.001 + extra
-    bad = err > tol
+    bad = ~(err <= tol)  # NaN is bad
     assert not bad.any(), f"{what}: {bad.sum()} of {bad.size} beyond tolerance; max err {err.max()}"
 
 
@@ -178,7 +183,7 @@ class AttnCase:
 
     def run(self, L, P):
         big = self.rng.standard_normal((L, self.stride)).astype(np.float16)
-        dbig, dQ, dout = dev(big), empty(HQ * L * HD * 2), empty(L * HQ * HD * 2)
+        dbig, dQ, dout = dev(big), unset(HQ * L * HD * 2), unset(L * HQ * HD * 2)
         self.sdamd.op_attention(dbig.data_ptr(), self.stride, self.dqw.data_ptr(), self.dkw.data_ptr(),
                                 self.drope.data_ptr(), L, P, HQ, HK, HD, self.rd, dQ.data_ptr(), self.dK.data_ptr(),
                                 self.dV.data_ptr(), CTX, dout.data_ptr())

@@ -33,7 +33,7 @@ def within_ulp(got, want, ulps=1.0, extra=0.0):
     want = np.asarray(want, np.float32)
     err = np.abs(got - want)
     tol = ulps * f16_ulp(want) * 1.001 + extra
-    bad = err > tol
+    bad = ~(err <= tol)  # NaN is bad
     assert not bad.any(), f"{bad.sum()} of {bad.size} beyond {ulps} f16 ulp; max err {err.max()}"
 
 
