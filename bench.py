@@ -315,7 +315,7 @@ def _algorithmic(cfg, seg, dispatches):
             b = L * d * (4 + 4 + 2 + 2) + 4 * d
         elif k.startswith("k_qk_prep"):  # q, gate-free k, v f16 in; Q, K, V f16 out
             b = 2 * L * (hq * hd + 2 * hk * hd) * 2
-        elif k.startswith("k_attn<"):  # Q, gate in; K, V of P + L keys; out f16
+        elif k.startswith(("k_attn<", "k_attn_rows<")):  # Q, gate in; K, V of P + L keys; out f16
             b = 2 * L * hq * hd * 3 + 2 * (P + L) * hk * hd * 2
         out.append((b, f))
     return out

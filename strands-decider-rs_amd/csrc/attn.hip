@@ -2,16 +2,15 @@
 // write (reference: src/kernels.rs:400-448), and causal GQA attention with a sigmoid output gate
 // (reference: src/kernels.rs:453-541).
 //
-// Attention runs on MFMA: k_attn for up to 128 rows, k_attn_rows above (attn_plan).  When the query
+// Attention runs on MFMA: k_attn for few rows, k_attn_rows for many (attn_plan).  When the query
 // blocks alone cannot fill the GPU (the short question suffix over a long cached prefix), the key range
-// is also split over workgroups and a combine kernel merges the partial (max, sum, acc).  As in the reference, q is pre-scaled
-// by 1/sqrt(hd) and rounded to f16 before the dot products.  The cache is kept in blocks of 32
+// is also split over workgroups and a combine kernel merges the partial (max, sum, acc).  As in the
+// reference, q is pre-scaled by 1/sqrt(hd) and rounded to f16 before the dot products.  The cache is kept in blocks of 32
 // keys, so that the fragment loads of a key block touch whole cache lines: K as [hk][ctx / 32]
 // [hd / 32][32 keys][32 dims] (a load of 16 keys x 8 dims reads pairs of consecutive keys' 64 bytes),
 // V transposed as [hk][ctx / 32][hd][32 keys] (a block's V^T is 16 KB of consecutive bytes).
 #include <climits>
 #include <cmath>
-#include <type_traits>
 
 #include "common.h"
 #include "device.h"
@@ -498,8 +497,8 @@ __global__ __launch_bounds__(256) void k_attn(const f16* __restrict__ Q, const f
 // v_mfma_f32_32x32x16_f16 where k_attn's feeds 16.  k_attn is bound by the CU's vector memory path (a
 // block is 32 KB per wave, 64 bytes a clock per CU) and by one wave per SIMD waiting in turn for its
 // loads, its softmax and its MFMAs.  This kernel is bound by that path too (2048 clocks for the four
-// waves' blocks, measured 2340 per block beside 1536 of MFMA), for twice the rows, plus about 15 thousand
-// clocks per workgroup of prologue and merge.  On MI355X, 8 query and 2 kv heads: 38.8 us at 2048 rows where
+// waves' blocks, measured 2340 per block beside 1536 of MFMA, which counters at 2048 rows show busy for 34%
+// of the CUs' cycles), for twice the rows, plus about 15 thousand clocks per workgroup of prologue and merge.  On MI355X, 8 query and 2 kv heads: 38.8 us at 2048 rows where
 // k_attn takes 104 us, 18.1 against 39 at 1024, 14.6 against 22.7 at 632; 440 TFLOP/s at 2048.
 //  * Row c of the workgroup is query c % NQ of head kh G + c / NQ; the 4 waves split the keys in blocks
 //    of 32 as in k_attn and merge their states in LDS at the end.
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(256) void k_attn(const f16* __restrict__ Q, const f
 //    block's as soon as its fragments have been read.  Rows of 64 bytes (a key's 32 dims of K, a dim's
 //    32 keys of V^T) have their 16-byte pieces at p ^ (row / 4) % 4, so a fragment read (32 rows, two
 //    pieces) meets no bank twice.
-//  * Per block: S^T = K Q^T (keys x rows, 16 MFMAs over the 256 dims in two chains), the softmax per
+//  * Per block: S^T = K Q^T (keys x rows, 16 MFMAs over the 256 dims in one chain), the softmax per
 //    column, O^T += V^T P^T (8 dim tiles x 2 key slices, P as f16 hi + lo).  The rows of S^T are permuted
 //    so that lane (column, half g) holds keys 16 s + 8 g .. + 7 in registers 8 s ..: P^T's B operand of
 //    slice s as it is.  Block n + 1's S MFMAs run among block n's exponentials.
@@ -996,9 +995,9 @@ size_t attn_ws_floats(int rows, const AttnShape& s) { return (size_t)ATTN_KS_MAX
 // Which kernel, and how many key splits, for L rows (prefix: the keys include a cached prefix; without one
 // they are the rows themselves).  The splits are fixed when a plan is captured, whatever the prefix's length.
 // qk_prep + attention + combine on MI355X at 8 query and 2 kv heads, us, k_attn against k_attn_rows:
-//   rows + prefix   64 + 512   120 + 512   200 + 512   250 + 2048   256 + 0   512 + 0   1024 + 0   2048 + 0
-//   k_attn          17.0       18.7        27.8        32.3         19.1      20.2      47.9       119
-//   k_attn_rows     18.4       19.3-20.6   22.3        29.4         16.1      19.0      26.7       51.1
+//   rows + prefix   64 + 512   120 + 512   200 + 512   250 + 2048   512 + 0   1024 + 0   2048 + 0
+//   k_attn          17.0       18.7        27.8        32.3         20.2      47.9       119
+//   k_attn_rows     18.4       19.3-20.6   22.3        29.4         19.0      26.7       51.1
 // A tile of 32 (query, head) rows has half as many workgroups as k_attn's 16 queries of a head, so up to 128
 // rows the latter's shorter chains win.  From 129 to 256 rows they also do (us, k_attn | k_attn_rows):
 //  * with few heads over a prefix, where 8 splits of k_attn are at most one workgroup per CU (32 tiles): 2

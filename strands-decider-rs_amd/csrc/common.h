@@ -243,7 +243,6 @@ struct AttnShape {
 // only (attention_split then computes the queries itself).
 void qk_prep(const f16* big, const AttnShape& s, const float* qw, const float* kw, const float* rope, int L,
              const uint32_t* lu, const Segs& sg, f16* Q, f16* Kc, f16* Vc, hipStream_t st);
-// Workspace (floats) of the key-split path for up to `rows` query rows and 8 splits.
 // How the attention of L query rows runs: the kernel (32 rows of all heads of a kv head per workgroup, or 16
 // queries of one head) and its key splits.  Only up to ATTN_SPLIT_ROWS rows split their keys.
 constexpr int ATTN_SPLIT_ROWS = 256;
@@ -253,6 +252,7 @@ struct AttnPlan {
     bool operator!=(const AttnPlan& o) const { return rows != o.rows || ks != o.ks; }
 };
 AttnPlan attn_plan(int L, const AttnShape& s, bool prefix);
+// Workspace (floats) of the key-split path for up to `rows` query rows and 8 splits.
 size_t attn_ws_floats(int rows, const AttnShape& s);
 // p.ks = number of key splits (1: no workspace needed; ks > 1 needs rows = L in the workspace).
 // Row r attends the prefix (cache rows < P) and its own sequence up to itself.

@@ -7,10 +7,6 @@
 namespace sd {
 namespace {
 
-// The 8 nibbles of a weight word in the engine nibble order (see k_repack_w4) as 4 f16 pairs q - 8
-// (exact) for k = (0,1), (2,3), (4,5), (6,7): the nibble at bits 4p lands in the f16 mantissa as
-// 1024 + q for p = 0, 2 (and 4, 6 in the high half), as 1024 + 16 q for the others, so two masks per
-// 8-bit shift give all four pairs.
 // Inline asm holds no vector instruction anywhere in these files: the compiler keeps the wait states
 // between an MFMA and a vector write of the registers it still reads as SrcC for its own instructions
 // only, not for those inside an asm.  Where it has to be led to one instruction, a constant or the
@@ -52,6 +48,10 @@ __device__ __forceinline__ float mul_add_f16(f16 h, float s, float b) {
     return r;
 }
 
+// The 8 nibbles of a weight word in the engine nibble order (see k_repack_w4) as 4 f16 pairs q - 8
+// (exact) for k = (0,1), (2,3), (4,5), (6,7): the nibble at bits 4p lands in the f16 mantissa as
+// 1024 + q for p = 0, 2 (and 4, 6 in the high half), as 1024 + 16 q for the others, so two masks per
+// 8-bit shift give all four pairs.
 __device__ __forceinline__ void nib_pairs(uint32_t w, f16x2& p0, f16x2& p1, f16x2& p2, f16x2& p3) {
     const uint32_t w8 = w >> 8;
     const f16x2 x0 = __builtin_bit_cast(f16x2, and_or(w, 0x000F000Fu, 0x64006400u));

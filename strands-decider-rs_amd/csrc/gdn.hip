@@ -168,10 +168,12 @@ constexpr int PREP_T = 512;  // k_gdn_prep threads: 8 waves
 // src/kernels.rs:152-170: rows before a sequence's start from the history, the prefix snapshot's when
 // lu names one); otherwise they are read from qkvc.
 // A workgroup is a chain of short phases, and a long input's many rounds also write 140 KB of operands a slot
-// (at 3000 rows two fifths to a half of the time at a copy's rate).  What lies above the diagonal of T, Qk and
-// Kn Kn^T is neither computed nor written where a whole tile of it does: 6 of 16 tiles of the products, 4 of 16 of
-// T's splits, 2 of 8 of Qk's fragments.  Whole op, with that work -> without, over two runs each: 17.1 -> 16.8 us at 65 rows,
-// 28.9 -> 28.6 at 512, 60.1 -> 59.3 at 1900.
+// (at 3000 rows two fifths to a half of the time at a copy's rate).  Above the diagonal of Kn Kn^T, Qn Kn^T and T
+// is left out what is whole tiles of a wave's step: 4 of 16 tiles of the products (the pairs 2, 3 of row tiles 0 and
+// 1, whose zeros still go to LDS; (0, 1) and (2, 3) are computed and masked), 4 of 16 of T's splits and their
+// products, 2 of 8 of Qk's fragments, which are not written either.  Whole op, with that work -> without, over two
+// runs each: 17.1 -> 16.8 us at 65 rows, 28.9 -> 28.6 at 512, 60.1 -> 59.3 at 1900.
+// (128 VGPRs, of which 8 or 10 go to scratch and come back once per chunk, around the inversion of T.)
 template <bool CONV>
 // Kernel arguments: the pointers and ints first, the structs last (the first 16 dwords are preloaded
 // into SGPRs, up to the first struct; the prologue needs the tables and big before anything else).
@@ -981,9 +983,10 @@ __global__ __launch_bounds__(RT) void k_gdn_recur(const uint32_t* __restrict__ l
 // clocks) and the chain of two LDS hand-offs; two workgroups per slice bring the former to 90 KB a chunk
 // (1900 tokens: 1.38 -> 0.97 us a chunk).
 // TWO: a grid of more than one workgroup per CU (several sequences, or many heads) is held to 128 VGPRs, so that
-// two fit on a CU: the next chunk's operands go to the registers of this one's as each is consumed.  The other form
-// has a second set for them, in 161 VGPRs, one workgroup per CU: 8 sequences of 25 tokens (1024 workgroups) 13.3 us
-// against 9.1 here, 3 of 40 (384) 7.7 against 5.5.
+// two fit on a CU: the next chunk's operands go to the registers of this one's as each is consumed (5 values that
+// only the end needs wait in scratch meanwhile; nothing inside the loop does).  The other form has a second set for
+// them, in 161 VGPRs, one workgroup per CU: 8 sequences of 25 tokens (1024 workgroups) 13.3 us against 9.1 here, 3
+// of 40 (384) 7.7 against 5.5.
 constexpr int SCAN_T = 512;
 template <bool TWO>
 __global__ __launch_bounds__(SCAN_T, TWO ? 4 : 2) void k_gdn_scan(const uint32_t* __restrict__ lu, const uint32_t* __restrict__ seqt,

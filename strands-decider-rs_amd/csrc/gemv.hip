@@ -291,8 +291,10 @@ __global__ __launch_bounds__(256) void k_gemv(const f16* __restrict__ A, const u
 //  * KH = 2: 8 waves, two k parts with their own rings, whose sums meet in LDS (a workgroup's chain of steps,
 //    which a short grid waits for, halves);
 //  * bound by each wave's chain of dequant (int3 asymmetric: about 190 VALU a step), fragment reads (every wave
-//    reads the whole A tile) and MFMAs: 15.5 us for the 2048 x 2048 matrix at 300 rows.  Pinning the dequant
-//    among the MFMAs with scheduling groups made it 21; 128 rows per workgroup 26.
+//    reads the whole A tile) and MFMAs, one after the other: 15.0 us for the 2048 x 2048 matrix at 300 rows, of
+//    whose CUs' cycles counters show the MFMAs busy for 24%, 2056 VALU instructions a wave (two waves a SIMD: about
+//    half of the issue), and one bank-conflict cycle for two of the fragment reads'.  Pinning the dequant among the
+//    MFMAs with scheduling groups made it 21; 128 rows per workgroup 26.
 template <int BITS>
 __device__ __forceinline__ void code_pairs(const typename BlkT<BITS>::T& w, int q, uint32_t (&p)[4]) {
     constexpr uint32_t EXP = 0x64006400u;  // f16 1024 in both halves: | q gives 1024 + q

@@ -72,9 +72,10 @@ def check(sdamd, o, seed, hq, hk, L, P, rd=64, gain=1.0, shift=0, own=False):
                            f"max {np.abs(got - want).max():.3g}")
 
 
-@pytest.mark.parametrize("L,P", [(129, 0), (136, 31), (150, 0), (159, 64), (193, 33), (256, 0), (257, 95), (264, 0), (300, 0), (513, 700)])
+@pytest.mark.parametrize("L,P", [(129, 0), (129, 31), (136, 31), (150, 0), (150, 40), (159, 64), (193, 33), (256, 0), (257, 95), (264, 0), (300, 0), (513, 700)])
 def test_rows_kernel_edges(sdamd, oracle, L, P):
-    """Ragged last tiles (8 queries each), prefixes that end inside a 32-key block, splits of 1, 2 and 4."""
+    """Ragged last tiles (8 queries each), prefixes that end inside a 32-key block, splits of 1, 2 and 4; without a
+    prefix the other kernel up to 256 rows."""
     check(sdamd, oracle, L + P, 8, 2, L, P)
 
 
